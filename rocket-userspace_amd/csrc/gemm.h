@@ -80,6 +80,10 @@ struct Launch {
 // N, K range and the problems' M only.
 size_t gemm_ws_bytes(const Launch &L);
 
+// Whether the launch takes the weight-streaming kernel of few rows (which converts fp32
+// operands as it loads them). Reads the formats, epilogue, K range and the problems' M only.
+bool gemm_streams(const Launch &L);
+
 // Validates the launch against what the kernels assume (alignment, sizes) and enqueues
 // it. Returns hipSuccess or an error; never faults on a rejected launch.
 hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out);

@@ -396,17 +396,6 @@ bool wide_tiles()
     return !e || atoi(e) != 0;
 }
 
-long row_bytes(Fmt f, int K)
-{
-    switch (f) {
-    case Fmt::I8: return K;
-    case Fmt::I4P: return K / 2;
-    case Fmt::I16: case Fmt::F16: case Fmt::BF16: return 2L * K;
-    case Fmt::F32BF16: case Fmt::F32TF32: case Fmt::BF16X2: return 4L * K;
-    }
-    return 0;
-}
-
 int stage_k(Fmt f) { return (f == Fmt::I8 || f == Fmt::I4P || f == Fmt::I16) ? 128 : 64; }
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
@@ -525,6 +514,17 @@ size_t ws_bytes_of(const Plan &p)
 
 }  // namespace
 
+long row_bytes(Fmt f, int K)
+{
+    switch (f) {
+    case Fmt::I8: return K;
+    case Fmt::I4P: return K / 2;
+    case Fmt::I16: case Fmt::F16: case Fmt::BF16: return 2L * K;
+    case Fmt::F32BF16: case Fmt::F32TF32: case Fmt::BF16X2: return 4L * K;
+    }
+    return 0;
+}
+
 // The family of a launch's operand formats and epilogue (one translation unit each).
 hipError_t dispatch(int bm, int bn, const Launch &L, const KArgs &ka, int blocks)
 {
@@ -546,7 +546,7 @@ size_t gemm_ws_bytes(const Launch &L)
         return 0;
     int maxM = 0;
     for (int i = 0; i < L.nprob; i++) maxM = std::max(maxM, L.prob[i].M);
-    if (maxM <= 0) return 0;
+    if (maxM <= 0 || stream_takes(L, maxM)) return 0;
     const Plan p = plan_of(L, maxM, true);
     return ws_bytes_of(p);
 }
@@ -557,6 +557,13 @@ void gemm_tile(Fmt fmt_a, Epi epi, int M, int N, int *bm, int *bn)
     const Choice c = choose(fmt_a, fmt_a, epi, M, 0, (long)M * N, false, tiles);
     *bm = c.bm;
     *bn = c.bn;
+}
+
+bool gemm_streams(const Launch &L)
+{
+    int maxM = 0;
+    for (int i = 0; i < L.nprob; i++) maxM = std::max(maxM, L.prob[i].M);
+    return maxM > 0 && stream_takes(L, maxM);
 }
 
 hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
@@ -611,12 +618,21 @@ hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
     }
     if (maxM == 0) return hipSuccess;
 
-    // a small fp16 product (whole K, one problem, few 32 x 32 blocks): the direct kernel
+    if (stream_takes(L, maxM)) {   // at most 16 rows
+        uint64_t blocks = 0;
+        const hipError_t e = stream_launch(L, &blocks);
+        if (blocks_out) *blocks_out = blocks;
+        return e;
+    }
+
+    // a small fp16 product (whole K, one problem, few 32 x 32 blocks, or one row of blocks, where
+    // the tiled kernels would fill a half or less of their rows: 16 x 512 x 8192 7.2 -> 4.0 us, 32 x 1024 x 8192 10.1 -> 7.6): the
+    // direct kernel
     if (L.fmt_a == Fmt::F16 && L.fmt_b == Fmt::F16 && (L.epi == Epi::F16 || L.epi == Epi::F32) && L.nprob == 1 &&
         !L.accum && L.kbeg == 0 && L.kend == L.K && L.K <= 1024) {
         const Problem &P = L.prob[0];
         const int nbm = (P.M + 31) / 32, nbn = (L.N + 31) / 32;
-        if ((long)nbm * nbn <= 64) {
+        if (nbm == 1 || (long)nbm * nbn <= 64) {
             const auto *A = static_cast<const _Float16 *>(P.A), *B = static_cast<const _Float16 *>(P.B);
             if (L.epi == Epi::F16)
                 hipLaunchKernelGGL(k_small_f16<true>, dim3(nbm * nbn), dim3(64), 0, L.stream, A, B, P.C, P.M, L.N, L.K, nbn);

@@ -1844,5 +1844,13 @@ hipError_t dispatch_gw_i4(int bm, int bn, const Launch &L, const KArgs &ka, int 
 hipError_t dispatch_f16(int bm, int bn, const Launch &L, const KArgs &ka, int blocks);    // fp16 operands
 hipError_t dispatch_bf16(int bm, int bn, const Launch &L, const KArgs &ka, int blocks);   // fp32 / bf16 / tf32 operands
 
+// HBM bytes of one operand row of K elements.
+long row_bytes(Fmt f, int K);
+
+// Products of at most 16 rows (stream.hip): whether the launch takes the weight-streaming
+// kernel, and its launch.
+bool stream_takes(const Launch &L, int maxM);
+hipError_t stream_launch(const Launch &L, uint64_t *blocks);
+
 }  // namespace gk
 }  // namespace rk

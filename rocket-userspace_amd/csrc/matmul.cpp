@@ -84,6 +84,11 @@ int f32_prepass(const Req &r)
     int maxM = 0;
     for (int p = 0; p < r.nprob; p++) maxM = std::max(maxM, r.M[p]);
     if (r.N < 256) return 0;
+    Launch L;   // few rows: the weight-streaming kernel converts as it loads
+    L.fmt_a = r.fa; L.fmt_b = r.fb; L.epi = r.epi; L.N = r.N; L.K = L.kend = r.K;
+    L.nprob = 1;
+    L.prob[0].M = maxM;
+    if (gemm_streams(L)) return 0;
     return (maxM >= 2048 && r.N >= 2048) ? 1 : 2;
 }
 
