@@ -49,6 +49,7 @@ struct Problem {
     const float *a_scale; // GW only: [M * nG]
     const float *b_scale; // GW only: [N * nG]
     const void *B2;       // GLU: the up weight [N/2, K]; ACT: fp16 bias [N] (or null)
+    const void *A2 = nullptr;   // quantised in the kernel (Launch::qa): the up rows, act(A) * A2
     // GW debug dump: the exact int32 partial of every K-group for rows [dump_row0,
     // dump_row0 + dump_rows), laid out [row][group][n] (null: none)
     int32_t *dump = nullptr;
@@ -63,7 +64,9 @@ struct Launch {
     int accum = 0;            // 1: add into C instead of overwriting it (chunked K)
     int group = 0;            // GW: quant group (elements of K)
     int rowscale = 0;         // GW: a_scale is one fp32 per row (Cf = a_scale[m] * sum_g fmaf(b_scale, P_g, .))
-    int act = 0;              // GLU / ACT: kActSilu or kActGelu
+    int act = 0;              // GLU / ACT, or qa with A2: kActSilu or kActGelu
+    int qa = 0;               // GW, rowscale: A holds fp32 (1) or fp16 (2) rows, quantised per row in the kernel
+                              // (quant_rows' formula; only where gemm_quantises says so)
     int f16out = 0;           // GW: C holds fp16 (each fp32 result rounded once) instead of fp32
     int kt = 0;               // GW: int32 partial period, divides group (== group normally)
     int nprob = 0;
@@ -83,6 +86,10 @@ size_t gemm_ws_bytes(const Launch &L);
 // Whether the launch takes the weight-streaming kernel of few rows (which converts fp32
 // operands as it loads them). Reads the formats, epilogue, K range and the problems' M only.
 bool gemm_streams(const Launch &L);
+
+// Whether a launch with `qa` set is one that quantises its rows itself (no quant_rows pass).
+// Reads the formats, epilogue, group, K range, the dump windows and the problems' M only.
+bool gemm_quantises(const Launch &L);
 
 // Validates the launch against what the kernels assume (alignment, sizes) and enqueues
 // it. Returns hipSuccess or an error; never faults on a rejected launch.

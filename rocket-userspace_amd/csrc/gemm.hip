@@ -151,38 +151,6 @@ struct QuantArgs {
     float *rs[kMaxProblems];
 };
 
-template <bool F16IN>
-__device__ __forceinline__ void load8f(const void *base, long i, float (&v)[8])
-{
-    if constexpr (F16IN) {
-        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-        const h8 h = *reinterpret_cast<const h8 *>(static_cast<const _Float16 *>(base) + i);
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = (float)h[e];
-    } else {
-        const f32x4 a = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + i);
-        const f32x4 b = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + i + 4);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            v[e] = a[e];
-            v[4 + e] = b[e];
-        }
-    }
-}
-
-__device__ __forceinline__ void quant_store8(int8_t *dst, const float (&v)[8], float s)
-{
-    uint32_t w[2] = {0u, 0u};
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        int q = (int)__builtin_rintf(v[e] * s);
-        q = q > 127 ? 127 : (q < -128 ? -128 : q);
-        w[e >> 2] |= (uint32_t)(q & 0xFF) << (8 * (e & 3));
-    }
-    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-    *reinterpret_cast<u2 *>(dst) = u2{w[0], w[1]};
-}
-
 // The 8 row values at element i of problem p: A's (ACT 0), or act(A) * A2 in fp32 (GLU).
 template <bool F16IN, int ACT>
 __device__ __forceinline__ void row8(const QuantArgs &qa, int p, long i, float (&v)[8])
@@ -566,6 +534,13 @@ bool gemm_streams(const Launch &L)
     return maxM > 0 && stream_takes(L, maxM);
 }
 
+bool gemm_quantises(const Launch &L)
+{
+    int maxM = 0;
+    for (int i = 0; i < L.nprob; i++) maxM = std::max(maxM, L.prob[i].M);
+    return L.qa && maxM > 0 && stream_gw_takes(L, maxM);
+}
+
 hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
 {
     if (blocks_out) *blocks_out = 0;
@@ -605,7 +580,8 @@ hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
         if (P.M == 0) continue;
         if (!P.A || !P.B || !P.C) return hipErrorInvalidValue;
         if (!aligned16(P.A) || !aligned16(P.B) || !aligned16(P.C)) return hipErrorInvalidValue;
-        if (L.epi == Epi::GW && (!P.a_scale || !P.b_scale)) return hipErrorInvalidValue;
+        if (L.epi == Epi::GW && ((!P.a_scale && !L.qa) || !P.b_scale)) return hipErrorInvalidValue;
+        if (L.qa && P.A2 && (!aligned16(P.A2) || (L.act != kActSilu && L.act != kActGelu))) return hipErrorInvalidValue;
         if (L.epi == Epi::GLU && (!P.B2 || !aligned16(P.B2))) return hipErrorInvalidValue;
         if (L.epi == Epi::ACT && P.B2 && ((uintptr_t)P.B2 & 1u)) return hipErrorInvalidValue;
         if (L.epi == Epi::GW && !L.rowscale && (long)P.M * nG * 4 >= (1L << 31)) return hipErrorInvalidValue;
@@ -621,6 +597,14 @@ hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
     if (stream_takes(L, maxM)) {   // at most 16 rows
         uint64_t blocks = 0;
         const hipError_t e = stream_launch(L, &blocks);
+        if (blocks_out) *blocks_out = blocks;
+        return e;
+    }
+
+    if (L.qa && !stream_gw_takes(L, maxM)) return hipErrorInvalidValue;
+    if (stream_gw_takes(L, maxM)) {   // at most 16 rows, group-wise
+        uint64_t blocks = 0;
+        const hipError_t e = stream_gw_launch(L, maxM, &blocks);
         if (blocks_out) *blocks_out = blocks;
         return e;
     }

@@ -336,6 +336,40 @@ template <int K> __device__ __forceinline__ float act_k(float x)
     else return x;   // kActIdentity
 }
 
+// Eight row values from element i on, as fp32.
+template <bool F16IN>
+__device__ __forceinline__ void load8f(const void *base, long i, float (&v)[8])
+{
+    if constexpr (F16IN) {
+        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+        const h8 h = *reinterpret_cast<const h8 *>(static_cast<const _Float16 *>(base) + i);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = (float)h[e];
+    } else {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + i);
+        const f32x4 b = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + i + 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v[e] = a[e];
+            v[4 + e] = b[e];
+        }
+    }
+}
+
+// Eight int8 codes rint(v * s), clamped, stored as 8 bytes.
+__device__ __forceinline__ void quant_store8(int8_t *dst, const float (&v)[8], float s)
+{
+    uint32_t w[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        int q = (int)__builtin_rintf(v[e] * s);
+        q = q > 127 ? 127 : (q < -128 ? -128 : q);
+        w[e >> 2] |= (uint32_t)(q & 0xFF) << (8 * (e & 3));
+    }
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    *reinterpret_cast<u2 *>(dst) = u2{w[0], w[1]};
+}
+
 // fp32 -> bf16 by truncation: the high halves of two fp32 words packed into one word.
 __device__ __forceinline__ int bf16pack(int f0, int f1)
 {
@@ -1851,6 +1885,9 @@ long row_bytes(Fmt f, int K);
 // kernel, and its launch.
 bool stream_takes(const Launch &L, int maxM);
 hipError_t stream_launch(const Launch &L, uint64_t *blocks);
+// The same for group-wise products of at most 16 rows (stream_gw.hip).
+bool stream_gw_takes(const Launch &L, int maxM);
+hipError_t stream_gw_launch(const Launch &L, int maxM, uint64_t *blocks);
 
 }  // namespace gk
 }  // namespace rk

@@ -118,13 +118,25 @@ int run(int fd, const Req &r)
     const size_t c_elem = r.f16out ? 2 : epi_elem_bytes(r.epi);
     const size_t a_row_in = qa_bytes ? qa_bytes * r.K : fmt_row_bytes(r.fa, r.K);
 
+    // few rows: the product quantises them itself (every launch of the call, or none)
+    bool fuse = qa_bytes != 0;
+    for (int p0 = 0; fuse && p0 < r.nprob; p0 += kMaxProblems) {
+        Launch Lq;
+        Lq.fmt_a = r.fa; Lq.fmt_b = fb_dev; Lq.epi = r.epi; Lq.N = r.N; Lq.K = Lq.kend = r.K;
+        Lq.group = r.group; Lq.kt = gw_period(r.group); Lq.rowscale = 1; Lq.qa = r.quant_a;
+        Lq.nprob = std::min(kMaxProblems, r.nprob - p0);
+        int rows = 0;
+        for (int q = 0; q < Lq.nprob; q++) rows += Lq.prob[q].M = r.M[p0 + q];
+        fuse = rows == 0 || gemm_quantises(Lq);
+    }
+
     Call c(L.h, r.who);
     for (int p = 0; p < r.nprob; p++) {
         const size_t M = (size_t)r.M[p];
         if (M == 0) continue;
         c.want(r.A[p], M * a_row_in);
         if (glu_in) c.want(r.A2[p], M * a_row_in);
-        if (qa_bytes) {
+        if (qa_bytes && !fuse) {
             c.want_scratch(M * r.K);
             c.want_scratch(M * sizeof(float));
         }
@@ -164,7 +176,7 @@ int run(int fd, const Req &r)
     for (int p0 = 0; p0 < r.nprob; p0 += kMaxProblems) {
         // the launch's activations quantised per row first (one pre-pass launch)
         QuantRows qr;
-        if (qa_bytes) {
+        if (qa_bytes && !fuse) {
             qr.n = std::min(kMaxProblems, r.nprob - p0);
             qr.K = r.K;
             qr.f16 = r.quant_a == 2;
@@ -200,6 +212,8 @@ int run(int fd, const Req &r)
         Lc.group = r.group;
         Lc.rowscale = r.rowscale;
         Lc.f16out = r.f16out ? 1 : 0;
+        Lc.qa = fuse ? r.quant_a : 0;
+        Lc.act = fuse ? r.act : 0;
         Lc.kt = gw ? gw_period(r.group) : 0;
         Lc.ws = wsp;
         Lc.ws_bytes = wsp ? ws : 0;
@@ -210,7 +224,11 @@ int run(int fd, const Req &r)
             P.M = r.M[p];
             P.B2 = nullptr;
             if (P.M == 0) { P.A = P.B = nullptr; P.C = nullptr; P.a_scale = P.b_scale = nullptr; continue; }
-            P.A = qa_bytes ? qr.Aq[q] : c.in(r.A[p], (size_t)P.M * fmt_row_bytes(r.fa, r.K));
+            P.A = qa_bytes && !fuse ? qr.Aq[q] : c.in(r.A[p], (size_t)P.M * a_row_in);
+            if (fuse && glu_in) {
+                P.A2 = c.in(r.A2[p], (size_t)P.M * a_row_in);
+                if (!P.A2) return c.finish();
+            }
             const void *b = c.in(r.B[p], (size_t)r.N * brow_in);
             if (r.pack_b_int4 && b) {
                 void *packed = c.scratch((size_t)r.N * r.K / 2);
@@ -236,12 +254,12 @@ int run(int fd, const Req &r)
                 }
             }
             P.C = c.out(r.C[p], (size_t)P.M * r.N * c_elem);
-            P.a_scale = !gw ? nullptr
+            P.a_scale = !gw || fuse ? nullptr
                         : qa_bytes ? qr.row_scale[q]
                                    : static_cast<const float *>(
                                          c.in(r.a_scale[p], (size_t)P.M * (r.rowscale ? 1 : nG) * sizeof(float)));
             P.b_scale = gw ? static_cast<const float *>(c.in(r.b_scale[p], (size_t)r.N * nG * sizeof(float))) : nullptr;
-            if (!P.A || !P.B || !P.C || (gw && (!P.a_scale || !P.b_scale))) return c.finish();
+            if (!P.A || !P.B || !P.C || (gw && ((!P.a_scale && !fuse) || !P.b_scale))) return c.finish();
             if (dump_of(p)) {
                 P.dump = static_cast<int32_t *>(c.out(dump_of(p), dump_bytes(p)));
                 P.dump_row0 = r.dump_row0[p];

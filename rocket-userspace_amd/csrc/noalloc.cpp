@@ -116,21 +116,6 @@ int rocket_matmul_int4_prepacked_gw_f32in_noalloc(rocket_i4_ctx *ctx, int M, int
     int8_t *Aq = reinterpret_cast<int8_t *>(base);
     float *rs = reinterpret_cast<float *>(base + codes);
 
-    QuantRows q;
-    q.n = 1;
-    q.K = K;
-    q.M[0] = M;
-    q.A[0] = A;
-    q.Aq[0] = Aq;
-    q.row_scale[0] = rs;
-    uint64_t blocks = 0;
-    if (quant_rows(q, L.h->stream, &blocks) != hipSuccess) {
-        (void)hipGetLastError();
-        ROCKET_LOGE("%s: quantisation launch rejected\n", who);
-        return ROCKET_E_SHAPE;
-    }
-    count_launch(blocks);
-
     Launch g;
     g.fmt_a = Fmt::I8;
     g.fmt_b = Fmt::I4P;
@@ -143,8 +128,28 @@ int rocket_matmul_int4_prepacked_gw_f32in_noalloc(rocket_i4_ctx *ctx, int M, int
     g.kt = gw_period(w->group);
     g.rowscale = 1;
     g.nprob = 1;
-    g.prob[0] = Problem{M, Aq, w->dev, Cf, rs, b_scale, nullptr};
+    g.prob[0] = Problem{M, A, w->dev, Cf, nullptr, b_scale, nullptr};
     g.stream = L.h->stream;
+    uint64_t blocks = 0;
+    g.qa = 1;
+    if (!gemm_quantises(g)) {   // more than a few rows: the codes and scales by a pass of their own
+        g.qa = 0;
+        QuantRows q;
+        q.n = 1;
+        q.K = K;
+        q.M[0] = M;
+        q.A[0] = A;
+        q.Aq[0] = Aq;
+        q.row_scale[0] = rs;
+        if (quant_rows(q, L.h->stream, &blocks) != hipSuccess) {
+            (void)hipGetLastError();
+            ROCKET_LOGE("%s: quantisation launch rejected\n", who);
+            return ROCKET_E_SHAPE;
+        }
+        count_launch(blocks);
+        g.prob[0].A = Aq;
+        g.prob[0].a_scale = rs;
+    }
     const hipError_t e = gemm_launch(g, &blocks);
     if (e != hipSuccess) {
         (void)hipGetLastError();
