@@ -65,6 +65,7 @@ struct FaArgs {
     int nsplit, tps;
     void *part;     // [split][head][T][dv] fp16 outputs, then [split][head][T] (max, sum) fp32 pairs
     int nqb;        // query blocks of BQ
+    int v_cols;     // readable columns of a V^T row (a multiple of 8): n_kv, or the padded row
 };
 
 // LDS per stage: the K tile (64 rows of DHP halves) then the V^T tile (DVP rows of 64 keys,
@@ -142,9 +143,11 @@ __global__ __launch_bounds__(256) void k_flash_attn(const FaArgs a)
     }
     // V^T: 8 chunks a row, so always separable (rows past dv are past the descriptor range)
     uint32_t vvo;
+    [[maybe_unused]] int vkey;   // the lane's chunk's first key in a tile (32 rows on: the same)
     {
         const int g = wave * 64 + lane, row = g >> 3, lc = (g & 7) ^ vx(row);
         vvo = (uint32_t)((long)row * a.v_rs + lc * 8) * 2u;
+        vkey = lc * 8;
     }
     const uint32_t kstep = (uint32_t)((256 / KCPR) * a.k_rs * 2), vstep = (uint32_t)(32 * a.v_rs * 2);
     const _Float16 *Kh = a.K + (size_t)hk * a.k_hs;
@@ -174,12 +177,15 @@ __global__ __launch_bounds__(256) void k_flash_attn(const FaArgs a)
         const long k0 = (long)kb * BK;
         const Rsrc rv = rsrc(Vh + k0, (uint32_t)((long)a.dv * a.v_rs * 2 - k0 * 2));
         char *vs = smem + slot * CF::STAGE + CF::KBYTES;
+        // rows of whole chunks (n_kv a multiple of 8) end where the last tile's chunks do: those past
+        // the row's end (the next row's keys) become zeros
+        const uint32_t past = k0 + vkey < a.v_cols ? 0u : kOOB;
 #pragma unroll
         for (int i = 0; i < VINS; i++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (__attribute__((address_space(3))) void *)(vs + (i * NW + wave) * 1024),
-                                                     16, vvo + i * vstep, 0, 0, 0);
+                                                     16, (vvo + i * vstep) | past, 0, 0, 0);
 #else
-        (void)kb; (void)slot; (void)vvo; (void)vstep;
+        (void)kb; (void)slot; (void)vvo; (void)vstep; (void)vkey;
 #endif
     };
 
@@ -564,14 +570,34 @@ __global__ __launch_bounds__(256) void k_fa_combine(const void *__restrict__ par
     }
 }
 
-__global__ void k_pad_cols(const _Float16 *__restrict__ src, long src_rs, _Float16 *__restrict__ dst, long rows,
-                           int cols, int cols_pad)
+// Eight output columns a thread (cols_pad a multiple of 8, dst 16-byte aligned): one unaligned
+// 16-byte load, one aligned store (a thread a column took 13 us for 2048 rows of 3000).
+struct __attribute__((packed, aligned(2))) Halves8 { f16x8 v; };
+// Rows [0, rows) come from src, the next rows2 from src2 (one launch for V and the mask).
+__global__ __launch_bounds__(256) void k_pad_cols(const _Float16 *__restrict__ src, _Float16 *__restrict__ dst, long rows,
+                                                  const _Float16 *__restrict__ src2, _Float16 *__restrict__ dst2, long rows2,
+                                                  int cols, int cols_pad)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * cols_pad) return;
-    const long r = i / cols_pad;
-    const int c = (int)(i % cols_pad);
-    dst[i] = c < cols ? src[r * src_rs + c] : (_Float16)0.f;
+    const int per = cols_pad / 8;
+    if (i >= (rows + rows2) * per) return;
+    long r = i / per;
+    const int c = (int)(i - r * per) * 8;
+    if (r >= rows) {
+        r -= rows;
+        src = src2;
+        dst = dst2;
+    }
+    const _Float16 *row = src + r * cols;
+    f16x8 v = {};
+    if (c + 8 <= cols) {
+        v = reinterpret_cast<const Halves8 *>(row + c)->v;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            if (c + e < cols) v[e] = row[c + e];
+    }
+    *reinterpret_cast<f16x8 *>(dst + r * cols_pad + c) = v;
 }
 
 __global__ void k_heads_transpose(const _Float16 *__restrict__ src, _Float16 *__restrict__ dst, int T, int n_head,
@@ -637,6 +663,7 @@ static int fa_splits(const FaLaunch &L)
 
 size_t flash_attn_ws_bytes(const FaLaunch &L)
 {
+    if (flash_attn_few_rows(L)) return flash_attn_rows_ws(L);
     const int ns = fa_splits(L);
     return ns > 1 ? (size_t)ns * L.n_head * L.T * (L.dv * sizeof(_Float16) + 2 * sizeof(float)) : 0;
 }
@@ -648,14 +675,16 @@ hipError_t flash_attn(const FaLaunch &L, hipStream_t s, uint64_t *blocks_out)
     if (L.dk < 16 || L.dk % 16 || L.dk > kAttnMaxHeadDim || L.dv < 16 || L.dv % 16 || L.dv > kAttnMaxHeadDim)
         return hipErrorInvalidValue;
     if (!L.Q || !L.K || !L.Vt || !L.O) return hipErrorInvalidValue;
-    // 16-byte Q / K chunks, 16-byte V^T DMA chunks, 8-byte output stores
+    // 16-byte Q / K chunks, 16-byte V^T DMA chunks (few rows: any V^T address), 8-byte output stores
+    const bool few = flash_attn_few_rows(L);
     if (!al(L.Q, 16) || !al(L.K, 16) || !al(L.Vt, 16) || !al(L.O, 8) || L.q_rs % 8 || L.q_hs % 8 || L.k_rs % 8 ||
-        L.k_hs % 8 || L.v_rs % 64 || L.v_hs % 8 || L.v_rs < L.n_kv || L.o_rs % 4 || L.o_hs % 4)
+        L.k_hs % 8 || (!few && ((L.v_rs % 64 && (L.v_rs % 8 || L.n_kv % 8)) || L.v_hs % 8)) || L.v_rs < L.n_kv || L.o_rs % 4 || L.o_hs % 4)
         return hipErrorInvalidValue;
     // buffer ranges and DMA offsets are 32-bit
     if ((long)L.n_kv * L.k_rs * 2 >= (1L << 31) || (long)L.dv * L.v_rs * 2 >= (1L << 31) ||
         (L.mask && ((long)L.T * L.m_rs * 2 >= (1L << 31) || L.m_rs < L.n_kv)))
         return hipErrorInvalidValue;
+    if (few) return flash_attn_rows(L, s, blocks_out);
     const bool mvec = L.mask && L.m_rs % 8 == 0 && al(L.mask, 16);
     FaArgs a;
     a.Q = L.Q; a.K = L.K; a.Vt = L.Vt; a.mask = L.mask; a.O = L.O;
@@ -663,6 +692,7 @@ hipError_t flash_attn(const FaLaunch &L, hipStream_t s, uint64_t *blocks_out)
     a.o_hs = L.o_hs; a.o_rs = L.o_rs; a.m_rs = L.m_rs;
     a.T = L.T; a.n_kv = L.n_kv; a.dk = L.dk; a.dv = L.dv; a.gqa = L.gqa; a.n_head = L.n_head;
     a.scale = L.scale; a.softcap = L.softcap;
+    a.v_cols = L.n_kv % 8 == 0 ? L.n_kv : (int)L.v_rs;
     const int tiles = (L.n_kv + BK - 1) / BK;
     a.nsplit = L.ws ? fa_splits(L) : 1;
     if (a.nsplit > 1 && L.ws_bytes < flash_attn_ws_bytes(L)) a.nsplit = 1;
@@ -713,13 +743,15 @@ hipError_t launch_fa_dims(const FaArgs &a, bool mvec, int dhp, int dvp, dim3 gri
 
 }  // namespace
 
-hipError_t pad_cols_f16(const _Float16 *src, long src_rs, _Float16 *dst, long rows, int cols, int cols_pad,
-                        hipStream_t s)
+hipError_t pad_cols_f16(const _Float16 *src, _Float16 *dst, long rows, const _Float16 *src2, _Float16 *dst2, long rows2, int cols,
+                        int cols_pad, hipStream_t s, uint64_t *blocks_out)
 {
-    if (rows < 1 || cols < 1 || cols_pad < cols || src_rs < cols) return hipErrorInvalidValue;
-    const long n = rows * cols_pad, blocks = (n + 255) / 256;
+    if (rows < 1 || rows2 < 0 || cols < 1 || cols_pad < cols || cols_pad % 8 || !al(dst, 16) || (rows2 && !al(dst2, 16)))
+        return hipErrorInvalidValue;
+    const long n = (rows + rows2) * (cols_pad / 8), blocks = (n + 255) / 256;
     if (blocks > 0x7FFFFFFFL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_pad_cols, dim3((unsigned)blocks), dim3(256), 0, s, src, src_rs, dst, rows, cols, cols_pad);
+    hipLaunchKernelGGL(k_pad_cols, dim3((unsigned)blocks), dim3(256), 0, s, src, dst, rows, src2, dst2, rows2, cols, cols_pad);
+    if (blocks_out) *blocks_out = (uint64_t)blocks;
     return hipGetLastError();
 }
 

@@ -42,11 +42,14 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     }
     const size_t nq = (size_t)n_head * T * dk, nk = (size_t)n_kv_heads * n_kv * dk;
     const size_t nv = (size_t)n_kv_heads * dv * n_kv, no = (size_t)n_head * T * dv, nm = (size_t)T * n_kv;
-    // V^T rows padded to a multiple of 64 keys (zeros) unless they already are
-    const int n_kvp = round_up(n_kv, 64);
-    const bool pad = n_kvp != n_kv;
     FaLaunch f;
     f.T = T; f.n_kv = n_kv; f.dk = dk; f.dv = dv; f.n_head = n_head; f.gqa = n_head / n_kv_heads;
+    // V^T rows are read in place by few query rows, and where they are whole 16-byte chunks; else
+    // they, and the mask's rows, are padded to a multiple of 64 keys (zeros), so that the mask's
+    // tiles too go by DMA (64 x 3001 keys, heads of 256: 46.0 us with a padding copy of a thread a
+    // value and the mask in 2-byte loads, 40.7 with eight values a thread, 28.2 with the mask too)
+    const int n_kvp = flash_attn_few_rows(f) || n_kv % 8 == 0 ? n_kv : round_up(n_kv, 64);
+    const bool pad = n_kvp != n_kv;
     f.scale = scale; f.softcap = softcap;
     const size_t ws = flash_attn_ws_bytes(f);
     Call c(L.h, who);
@@ -57,6 +60,8 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     if (mask) c.want(mask, h16(nm));
     c.want(out, h16(no));
     if (pad) c.want_scratch(h16((size_t)n_kv_heads * dv * n_kvp));
+    const bool pad_m = pad && mask && (size_t)T * n_kvp < ((size_t)1 << 30);   // (32-bit offsets into it)
+    if (pad_m) c.want_scratch(h16((size_t)T * n_kvp));
     if (int rc = c.begin()) return rc;
     f.ws = ws ? static_cast<float *>(c.scratch(ws)) : nullptr;
     f.ws_bytes = f.ws ? ws : 0;
@@ -68,14 +73,17 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     if (!f.Q || !f.K || !dV || (mask && !f.mask) || !f.O) return c.finish();
     if (pad) {
         _Float16 *vp = static_cast<_Float16 *>(c.scratch(h16((size_t)n_kv_heads * dv * n_kvp)));
-        if (!vp) return c.finish();
-        if (pad_cols_f16(dV, n_kv, vp, (long)n_kv_heads * dv, n_kv, n_kvp, c.stream()) != hipSuccess) {
+        _Float16 *mp = pad_m ? static_cast<_Float16 *>(c.scratch(h16((size_t)T * n_kvp))) : nullptr;
+        if (!vp || (pad_m && !mp)) return c.finish();
+        uint64_t pb = 0;
+        if (pad_cols_f16(dV, vp, (long)n_kv_heads * dv, f.mask, mp, pad_m ? T : 0, n_kv, n_kvp, c.stream(), &pb) != hipSuccess) {
             (void)hipGetLastError();
             ROCKET_LOGE("%s: V pad launch rejected\n", who);
             (void)c.finish();
             return ROCKET_E_DEVICE;
         }
-        count_launch((uint64_t)(((size_t)n_kv_heads * dv * n_kvp + 255) / 256));
+        count_launch(pb);
+        if (pad_m) f.mask = mp;
         dV = vp;
     }
     f.Vt = dV;
@@ -83,7 +91,7 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     f.k_hs = (long)n_kv * dk; f.k_rs = dk;
     f.v_hs = (long)dv * n_kvp; f.v_rs = n_kvp;
     f.o_hs = (long)T * dv; f.o_rs = dv;
-    f.m_rs = n_kv;
+    f.m_rs = pad_m ? n_kvp : n_kv;
     uint64_t blocks = 0;
     if (flash_attn(f, c.stream(), &blocks) != hipSuccess) {
         (void)hipGetLastError();
