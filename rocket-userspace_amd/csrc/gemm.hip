@@ -6,6 +6,8 @@
 // and K slices, and calls the family's dispatcher.
 #include "gemm_impl.h"
 
+#include <cmath>
+
 namespace rk {
 namespace gk {
 namespace {
@@ -432,6 +434,72 @@ Choice choose(Fmt fa, Fmt fb, Epi epi, int maxM, int kspan, long outs, bool accu
     return {64, 64, 1};
 }
 
+// Products of fp16 / fp32 operands whose tiles leave the GPU waiting for one workgroup's chain of
+// stages: K in slices of smaller tiles, by estimated time. A stage takes its latency, or, with n
+// workgroups on a CU, the n stages' operand bytes at 58 KB / us or their MFMAs, whichever is
+// longest; slices add a launch and their planes' bytes. The constants are fits to 40 products of 24
+// to 1024 rows, every tile and slice count timed (the estimate's choice took at most 1.2 times the
+// fastest, but for a 24-row one of 12 us); us and KB.
+struct StageFit {
+    int bm, bn;
+    double lat;   // a stage alone on its CU
+    int res;      // workgroups of it that a CU holds
+};
+constexpr StageFit kFitF16[] = {{64, 64, 0.31, 5}, {128, 64, 0.34, 2}, {128, 128, 0.8, 2}, {256, 128, 1.0, 1}};
+constexpr StageFit kFitBF16[] = {{64, 64, 0.38, 5}, {128, 64, 0.45, 2}, {128, 128, 0.85, 2}, {256, 128, 1.1, 1}};
+constexpr StageFit kFitTF32[] = {{64, 64, 0.62, 2}, {128, 64, 0.75, 1}, {128, 128, 1.4, 1}};
+
+struct FloatMath {
+    const StageFit *fit;
+    int n;
+    double ea, eb, mflop;   // bytes of an A and a B element as the tiles load them; MFLOP a us and CU
+    double fixed;           // launches: the product's, and the conversion of A's
+};
+
+FloatMath float_math(Fmt fa)
+{
+    if (fa == Fmt::F16) return {kFitF16, 4, 2, 2, 5.0, 2.5};
+    if (fa == Fmt::F32BF16 || fa == Fmt::BF16) return {kFitBF16, 4, 2, 4, 5.0, 5.5};
+    return {kFitTF32, 3, 4, 4, 1.75, 5.5};
+}
+
+double plan_time(const FloatMath &m, const StageFit &f, int M, int K, int N, int slices)
+{
+    const int nst = (K + 63) / 64, per = (nst + slices - 1) / slices, z = (nst + per - 1) / per;
+    const long wgs = (long)((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn) * z;
+    const double n = (double)((wgs + 255) / 256);
+    const double kb = (f.bm * m.ea + f.bn * m.eb) * 64 / 1000, mf = f.bm * (double)f.bn * 128e-6 / m.mflop;
+    double t = per * std::max(f.lat * std::ceil(n / f.res), n * std::max(kb / 58, mf));
+    t = std::max(t, ((double)M * K * m.ea + (double)N * K * m.eb) / 4.8e6);
+    if (z > 1) t += 3.0 + (double)z * M * N * 4 * (1 / 6.5e6 + 1 / 5e6);
+    return m.fixed + t;
+}
+
+// The estimate's choice for one product, where it takes at most 0.85 of the time of `base` (the choice
+// of choose() on unconverted operands, so that converting them first changes no slicing). A plain
+// fp16 row keeps the bits that one chain over K gives it, whatever M and N, up to K = 2048.
+bool choose_slices(Fmt fa, int M, int K, int N, const Choice &base, Choice *out)
+{
+    if (base.bn == 256) return false;
+    const FloatMath m = float_math(fa);
+    const char *env = getenv("ROCKET_HIP_SPLITK");
+    const int cap = env ? splitk_cap() : 8, most = fa == Fmt::F16 && K <= 2048 ? 1 : cap;
+    double now = 0, best = 0;
+    for (int i = 0; i < m.n; i++) {
+        const StageFit &f = m.fit[i];
+        if (f.bm == base.bm && f.bn == base.bn) now = plan_time(m, f, M, K, N, base.splitk);
+        for (int z = 1; z <= most; z *= 2) {
+            if (z > 1 && K / z < 256) break;
+            const double t = plan_time(m, f, M, K, N, z);
+            if (best == 0 || t < best) {
+                best = t;
+                *out = Choice{f.bm, f.bn, z};
+            }
+        }
+    }
+    return now > 0 && best <= 0.85 * now;
+}
+
 // Tile geometry and K slices of a launch whose largest problem has maxM rows. Slices cover
 // whole stages and none is empty.
 struct Plan {
@@ -456,7 +524,14 @@ Plan plan_of(const Launch &L, int maxM, bool allow_split)
     const bool split_ok = allow_split && L.nprob == 1 && (L.epi == Epi::I32 || (fp && !L.accum));
     long outs = 0;
     for (int i = 0; i < L.nprob; i++) outs += (long)L.prob[i].M * L.N;
-    const Choice c = choose(L.fmt_a, L.fmt_b, L.epi, maxM, kspan, outs, split_ok, tiles);
+    Choice c = choose(L.fmt_a, L.fmt_b, L.epi, maxM, kspan, outs, split_ok, tiles);
+    // (large tiles that cover the CUs in one chain over K are left alone, without an estimate)
+    if (split_ok && fp && kspan == L.K && !(c.splitk == 1 && c.bm >= 128 && tiles(c.bm, c.bn) >= 240)) {
+        const Fmt raw = L.fmt_a == Fmt::BF16 ? Fmt::F32BF16 : L.fmt_a == Fmt::BF16X2 ? Fmt::F32TF32 : L.fmt_a;
+        const Choice base = choose(raw, raw, L.epi, maxM, kspan, outs, split_ok, tiles);
+        Choice x;
+        if (choose_slices(L.fmt_a, maxM, L.K, L.N, base, &x)) c = x;
+    }
     Plan p;
     p.bm = c.bm;
     p.bn = c.bn;
@@ -471,6 +546,17 @@ Plan plan_of(const Launch &L, int maxM, bool allow_split)
     p.m0 = L.prob[0].M;
     p.n = L.N;
     return p;
+}
+
+// A small fp16 product (whole K, one problem, few 32 x 32 blocks, or one row of blocks, where the
+// tiled kernels would fill a half or less of their rows: 16 x 512 x 8192 7.2 -> 4.0 us, 32 x 1024 x
+// 8192 10.1 -> 7.6): the direct kernel.
+bool small_takes(const Launch &L, int maxM)
+{
+    if (L.fmt_a != Fmt::F16 || L.fmt_b != Fmt::F16 || (L.epi != Epi::F16 && L.epi != Epi::F32) || L.nprob != 1 || L.accum ||
+        L.kbeg != 0 || L.kend != L.K || L.K > 1024)
+        return false;
+    return maxM <= 32 || (long)((maxM + 31) / 32) * ((L.N + 31) / 32) <= 64;
 }
 
 // [slice][M][N] planes of fp32 partials
@@ -514,7 +600,7 @@ size_t gemm_ws_bytes(const Launch &L)
         return 0;
     int maxM = 0;
     for (int i = 0; i < L.nprob; i++) maxM = std::max(maxM, L.prob[i].M);
-    if (maxM <= 0 || stream_takes(L, maxM)) return 0;
+    if (maxM <= 0 || stream_takes(L, maxM) || small_takes(L, maxM)) return 0;   // (no slices: no planes)
     const Plan p = plan_of(L, maxM, true);
     return ws_bytes_of(p);
 }
@@ -609,22 +695,16 @@ hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
         return e;
     }
 
-    // a small fp16 product (whole K, one problem, few 32 x 32 blocks, or one row of blocks, where
-    // the tiled kernels would fill a half or less of their rows: 16 x 512 x 8192 7.2 -> 4.0 us, 32 x 1024 x 8192 10.1 -> 7.6): the
-    // direct kernel
-    if (L.fmt_a == Fmt::F16 && L.fmt_b == Fmt::F16 && (L.epi == Epi::F16 || L.epi == Epi::F32) && L.nprob == 1 &&
-        !L.accum && L.kbeg == 0 && L.kend == L.K && L.K <= 1024) {
+    if (small_takes(L, maxM)) {
         const Problem &P = L.prob[0];
         const int nbm = (P.M + 31) / 32, nbn = (L.N + 31) / 32;
-        if (nbm == 1 || (long)nbm * nbn <= 64) {
-            const auto *A = static_cast<const _Float16 *>(P.A), *B = static_cast<const _Float16 *>(P.B);
-            if (L.epi == Epi::F16)
-                hipLaunchKernelGGL(k_small_f16<true>, dim3(nbm * nbn), dim3(64), 0, L.stream, A, B, P.C, P.M, L.N, L.K, nbn);
-            else
-                hipLaunchKernelGGL(k_small_f16<false>, dim3(nbm * nbn), dim3(64), 0, L.stream, A, B, P.C, P.M, L.N, L.K, nbn);
-            if (blocks_out) *blocks_out = (uint64_t)nbm * nbn;
-            return hipGetLastError();
-        }
+        const auto *A = static_cast<const _Float16 *>(P.A), *B = static_cast<const _Float16 *>(P.B);
+        if (L.epi == Epi::F16)
+            hipLaunchKernelGGL(k_small_f16<true>, dim3(nbm * nbn), dim3(64), 0, L.stream, A, B, P.C, P.M, L.N, L.K, nbn);
+        else
+            hipLaunchKernelGGL(k_small_f16<false>, dim3(nbm * nbn), dim3(64), 0, L.stream, A, B, P.C, P.M, L.N, L.K, nbn);
+        if (blocks_out) *blocks_out = (uint64_t)nbm * nbn;
+        return hipGetLastError();
     }
 
     Plan pl = plan_of(L, maxM, true);

@@ -70,7 +70,7 @@ int gw_period(int group)
 // converted first in one streaming pass into the handle's arena (bf16: half the bytes;
 // tf32: hi/lo pairs), so the GEMM moves half the bytes through L2 (bf16) and spends no VALU
 // on the conversion. The pass costs one extra read + write of the operand, so it pays for
-// an operand whose rows many tiles re-read: A (read once per 128-column tile) from N >= 256,
+// an operand whose rows many tiles re-read: A (read once per 128-column tile) from N >= 384,
 // B (read once per 256-row tile) from M >= 2048 (measured on MI355X: A alone is 5-25%
 // faster than neither from M = 64 up; both are 1.4-2.3x faster from M = 2048 up, A alone
 // up to M = 1024). Returns 0 (no pass), 1 (both operands) or 2 (A only).
@@ -83,7 +83,10 @@ int f32_prepass(const Req &r)
     }
     int maxM = 0;
     for (int p = 0; p < r.nprob; p++) maxM = std::max(maxM, r.M[p]);
-    if (r.N < 256) return 0;
+    // (with few columns, or few values, the pass's own launch costs more than it saves: tf32 700 x
+    // 2528 x 272 25.6 us with it, 20.3 without; 128 x 2048 x 2048 17.5 and 16.0; 128 x 4096 x 4096
+    // 30.6 and 33.4)
+    if (r.N < 384 || (long)maxM * r.K < 400000) return 0;
     Launch L;   // few rows: the weight-streaming kernel converts as it loads
     L.fmt_a = r.fa; L.fmt_b = r.fb; L.epi = r.epi; L.N = r.N; L.K = L.kend = r.K;
     L.nprob = 1;
