@@ -387,7 +387,11 @@ Choice choose(Fmt fa, Fmt fb, Epi epi, int maxM, int kspan, long outs, bool accu
         // one workgroup per CU) when the rows fill it and it still gives most CUs a tile.
         if (maxM > 128 && tiles(256, 128) >= cus * 3 / 4) return {256, 128, 1};
         if (tiles(128, 128) >= cus * 3 / 4) return {128, 128, 1};
-        if (tiles(128, 64) >= cus / 2) return {128, 64, 1};
+        // 128 x 64 against int8 weights from half the CUs (grouped products of 351 tokens, 3456 -> 672:
+        // 52.9 us, 64 x 64 57.3), against int4 from all of them (64 x 64 with up to two workgroups a CU:
+        // 256 x 4096 x 4096 in groups of 32 44.3 -> 31.3 us, 412 x 6880 x 2688 68.6 -> 54.1, 116 x 1952 x
+        // 16192 31.3 -> 27.2)
+        if (tiles(128, 64) >= (fb == Fmt::I4P ? cus : cus / 2)) return {128, 64, 1};
         return {64, 64, 1};
     }
     if (epi == Epi::I32) {
@@ -695,6 +699,12 @@ hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
         return e;
     }
 
+    if (mid_gw_takes(L, maxM)) {   // 17 rows and more, group-wise, as long as the workgroups fit the GPU
+        uint64_t blocks = 0;
+        const hipError_t e = mid_gw_launch(L, maxM, &blocks);
+        if (blocks_out) *blocks_out = blocks;
+        return e;
+    }
     if (small_takes(L, maxM)) {
         const Problem &P = L.prob[0];
         const int nbm = (P.M + 31) / 32, nbn = (L.N + 31) / 32;

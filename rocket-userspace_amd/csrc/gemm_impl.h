@@ -1888,6 +1888,9 @@ hipError_t stream_launch(const Launch &L, uint64_t *blocks);
 // The same for group-wise products of at most 16 rows (stream_gw.hip).
 bool stream_gw_takes(const Launch &L, int maxM);
 hipError_t stream_gw_launch(const Launch &L, int maxM, uint64_t *blocks);
+// The same for 17 rows and more, up to what fits the GPU at once (stream_gw_mid.hip).
+bool mid_gw_takes(const Launch &L, int maxM);
+hipError_t mid_gw_launch(const Launch &L, int maxM, uint64_t *blocks);
 
 }  // namespace gk
 }  // namespace rk
