@@ -51,9 +51,7 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     const int n_kvp = flash_attn_few_rows(f) || n_kv % 8 == 0 ? n_kv : round_up(n_kv, 64);
     const bool pad = n_kvp != n_kv;
     f.scale = scale; f.softcap = softcap;
-    const size_t ws = flash_attn_ws_bytes(f);
     Call c(L.h, who);
-    if (ws) c.want_scratch(ws);
     c.want(Q, h16(nq));
     c.want(K, h16(nk));
     c.want(V, h16(nv));
@@ -62,6 +60,7 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     if (pad) c.want_scratch(h16((size_t)n_kv_heads * dv * n_kvp));
     const bool pad_m = pad && mask && (size_t)T * n_kvp < ((size_t)1 << 30);   // (32-bit offsets into it)
     if (pad_m) c.want_scratch(h16((size_t)T * n_kvp));
+    const size_t ws = c.want_optional(flash_attn_ws_bytes(f));
     if (int rc = c.begin()) return rc;
     f.ws = ws ? static_cast<float *>(c.scratch(ws)) : nullptr;
     f.ws_bytes = f.ws ? ws : 0;

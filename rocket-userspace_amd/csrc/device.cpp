@@ -223,6 +223,18 @@ void Call::want(const void *p, size_t bytes)
     if (!direct_(p)) need_ += round_(bytes);
 }
 
+size_t Call::want_optional(size_t bytes)
+{
+    if (bytes == 0) return 0;
+    if (need_ + round_(bytes) > h_->arena_cap) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(h_->stream, &cap) != hipSuccess) (void)hipGetLastError();
+        if (cap != hipStreamCaptureStatusNone) return 0;
+    }
+    want_scratch(bytes);
+    return bytes;
+}
+
 int Call::begin()
 {
     PhaseTimer pt(t_stage_);

@@ -58,6 +58,10 @@ public:
     // Reserve arena space before in()/out(): sum of every host operand's bytes.
     void want(const void *p, size_t bytes);
     void want_scratch(size_t bytes) { need_ += round_(bytes); }
+    // Scratch that the launch can do without (K slices' planes): `bytes`, reserved, or 0 where the
+    // arena would have to grow while the handle's stream is being captured, which allows no
+    // allocation. The last of the reservations.
+    size_t want_optional(size_t bytes);
     int  begin();                          // grows the arena if needed
     void *in(const void *p, size_t bytes);  // device view of an input
     void *out(void *p, size_t bytes);       // device view of an output

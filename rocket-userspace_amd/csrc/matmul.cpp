@@ -66,6 +66,21 @@ int gw_period(int group)
     return 32;
 }
 
+// Whether a result of the call lies over rows (A, A2) of it.
+bool results_overlap_rows(const Req &r, size_t a_row, size_t c_elem)
+{
+    const auto over = [](const void *a, size_t na, const void *c, size_t nc) {
+        const uintptr_t x = (uintptr_t)a, y = (uintptr_t)c;
+        return x < y + nc && y < x + na;
+    };
+    for (int p = 0; p < r.nprob; p++)
+        for (int q = 0; q < r.nprob; q++) {
+            const size_t na = (size_t)r.M[p] * a_row, nc = (size_t)r.M[q] * r.N * c_elem;
+            if (na && nc && (over(r.A[p], na, r.C[q], nc) || (r.A2 && over(r.A2[p], na, r.C[q], nc)))) return true;
+        }
+    return false;
+}
+
 // fp32 operands (bf16 / tf32 entries) are either converted as the GEMM loads them, or
 // converted first in one streaming pass into the handle's arena (bf16: half the bytes;
 // tf32: hi/lo pairs), so the GEMM moves half the bytes through L2 (bf16) and spends no VALU
@@ -86,12 +101,14 @@ int f32_prepass(const Req &r)
     // (with few columns, or few values, the pass's own launch costs more than it saves: tf32 700 x
     // 2528 x 272 25.6 us with it, 20.3 without; 128 x 2048 x 2048 17.5 and 16.0; 128 x 4096 x 4096
     // 30.6 and 33.4)
-    if (r.N < 384 || (long)maxM * r.K < 400000) return 0;
+    bool pays = r.N >= 384 && (long)maxM * r.K >= 400000;
     Launch L;   // few rows: the weight-streaming kernel converts as it loads
     L.fmt_a = r.fa; L.fmt_b = r.fb; L.epi = r.epi; L.N = r.N; L.K = L.kend = r.K;
     L.nprob = 1;
     L.prob[0].M = maxM;
-    if (gemm_streams(L)) return 0;
+    if (pays) pays = !gemm_streams(L);
+    // (results stored over the rows: with the pass every row has been read before the first of them)
+    if (!pays) return r.N >= 256 && results_overlap_rows(r, (size_t)r.K * 4, 4) ? 2 : 0;
     return (maxM >= 2048 && r.N >= 2048) ? 1 : 2;
 }
 
@@ -132,6 +149,8 @@ int run(int fd, const Req &r)
         for (int q = 0; q < Lq.nprob; q++) rows += Lq.prob[q].M = r.M[p0 + q];
         fuse = rows == 0 || gemm_quantises(Lq);
     }
+    // (a pass of its own has read every row before the first result is stored)
+    if (fuse && results_overlap_rows(r, a_row_in, c_elem)) fuse = false;
 
     Call c(L.h, r.who);
     for (int p = 0; p < r.nprob; p++) {
@@ -170,7 +189,7 @@ int run(int fd, const Req &r)
             Lp.kend = (r.kchunk > 0 && r.K > r.kchunk) ? r.kchunk : r.K;
             ws = std::max(ws, gemm_ws_bytes(Lp));
         }
-        c.want_scratch(ws);
+        ws = c.want_optional(ws);
     }
     if (int rc = c.begin()) return rc;
     int32_t *wsp = ws ? static_cast<int32_t *>(c.scratch(ws)) : nullptr;

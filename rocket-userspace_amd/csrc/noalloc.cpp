@@ -12,9 +12,9 @@
 // the array. Nothing in it needs clearing: the pre-pass writes every code and scale the GEMM
 // reads.
 //
-// Under HIP graph capture of the handle's stream the entry only records its two launches: it
-// neither waits for them (stream queries and synchronisation are illegal while a stream
-// captures) nor drains a handle left dirty by an earlier wait that gave up (that case is
+// Under HIP graph capture of the handle's stream the entry only records its launches (two, or
+// one for few rows): it neither waits for them (stream queries and synchronisation are illegal
+// while a stream captures) nor drains a handle left dirty by an earlier wait that gave up (that case is
 // refused, since draining would invalidate the capture). A replayed graph writes Cf when it
 // runs. Nothing it records is a memset or a copy.
 #include "ops.h"
@@ -132,7 +132,9 @@ int rocket_matmul_int4_prepacked_gw_f32in_noalloc(rocket_i4_ctx *ctx, int M, int
     g.stream = L.h->stream;
     uint64_t blocks = 0;
     g.qa = 1;
-    if (!gemm_quantises(g)) {   // more than a few rows: the codes and scales by a pass of their own
+    const bool over = (uintptr_t)A < (uintptr_t)Cf + (size_t)M * N * 4 && (uintptr_t)Cf < (uintptr_t)A + (size_t)M * K * 4;
+    // more than a few rows, or results over them: the codes and scales by a pass of their own
+    if (over || !gemm_quantises(g)) {
         g.qa = 0;
         QuantRows q;
         q.n = 1;

@@ -1,0 +1,116 @@
+"""Calls whose results lie over their own rows, and calls recorded into a HIP graph on a handle that
+has no scratch yet, on the GPU: rows that a pass of their own reads (quantised fp32 rows, converted
+fp32 operands) are all read before the first result is stored, for few rows as for many; and a
+product or an attention that would take scratch for K slices or key splits runs without them."""
+import numpy as np
+import pytest
+
+import rocketnpu as R
+
+pytestmark = pytest.mark.gpu
+SEED = 0x52434F80
+DEV = "cuda:0"
+
+
+def _handle(lib, fd, stream):
+    assert lib.rocket_hip_set_stream(fd, R.ptr(stream.cuda_stream)) == 0
+    assert lib.rocket_hip_set_mode(fd, R.ROCKET_HIP_ASYNC | R.ROCKET_HIP_DEVICE_OPERANDS) == 0
+
+
+@pytest.mark.parametrize("M", [4, 16, 64])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_quantised_rows_under_results(lib, orc, M, noalloc):
+    import torch
+    K = N = 1024
+    group = 128
+    print(f"quantised rows under results M={M} noalloc={noalloc}", flush=True)
+    B = orc.gen_i8((N, K), SEED + 1, -8, 7)
+    bsc = orc.gen_uniform((N, K // group), SEED + 2, 0.005, 0.02)
+    x = orc.gen_normal((M, K), SEED + 3)
+    ctx = lib.rocket_i4_ctx_create(1)
+    w = lib.rocket_i4_weights_pack_gw(ctx, M, K, N, R.ptr(B), group)
+    assert w
+    fn = getattr(lib, "rocket_matmul_int4_prepacked_gw_f32in" + ("_noalloc" if noalloc else ""))
+    q, s = orc.quant_rows(x)
+    want = orc.matmul_gw_rowscale_f32(q, B, s, bsc, group)
+    stream = torch.cuda.Stream()
+    _handle(lib, lib.rocket_i4_ctx_fd(ctx), stream)
+    with torch.cuda.stream(stream):
+        dx, dbs = torch.from_numpy(x).to(DEV), torch.from_numpy(bsc).to(DEV)
+        assert fn(ctx, M, K, N, R.ptr(dx), R.ptr(dbs), R.ptr(dx), w) == 0
+        got = dx.cpu().numpy()
+    assert np.array_equal(got, want)
+    lib.rocket_i4_weights_free(ctx, w)
+    lib.rocket_i4_ctx_free(ctx)
+
+
+@pytest.mark.parametrize("M", [4, 16, 64, 300])
+@pytest.mark.parametrize("math", ["bf16", "tf32"])
+def test_converted_rows_under_results(lib, orc, M, math):
+    import torch
+    K = N = 512
+    print(f"converted rows under results M={M} {math}", flush=True)
+    x, B = orc.gen_normal((M, K), SEED + 4), orc.gen_normal((N, K), SEED + 5)
+    fd = lib.rocket_open()
+    stream = torch.cuda.Stream()
+    _handle(lib, fd, stream)
+    fn = getattr(lib, "rocket_matmul_" + math)
+    # both operands truncated to the entry's mantissa, products exact in fp32, sums of K terms
+    cut = np.uint32(0xFFFF0000 if math == "bf16" else 0xFFFFE000)
+    t = lambda a: (a.view(np.uint32) & cut).view(np.float32).astype(np.float64)  # noqa: E731
+    want, mag = t(x) @ t(B).T, np.abs(t(x)) @ np.abs(t(B)).T
+    with torch.cuda.stream(stream):
+        dx, dB = torch.from_numpy(x).to(DEV), torch.from_numpy(B).to(DEV)
+        assert fn(fd, M, K, N, R.ptr(dx), R.ptr(dB), R.ptr(dx)) == 0
+        got = dx.cpu().numpy().astype(np.float64)
+    # three products a term at tf32: (3 K + 1) roundings of 2^-24 of the terms' magnitudes at most
+    assert np.all(np.abs(got - want) <= (3 * K + 1) * 2.0 ** -24 * mag)
+    lib.rocket_close(fd)
+
+
+@pytest.mark.parametrize("op", ["fp16", "attn"])
+def test_capture_on_a_fresh_handle(lib, orc, monkeypatch, op):
+    import torch
+    print(f"capture on a fresh handle {op}", flush=True)
+    stream = torch.cuda.Stream()
+    h = lambda shape, k, sc=1.0: torch.from_numpy((orc.gen_normal(shape, SEED + k) * sc).astype(np.float16)).to(DEV)  # noqa: E731
+    if op == "fp16":
+        M, K, N = 64, 4096, 1024
+        a, b = h((M, K), 6), h((N, K), 7)
+        out = torch.empty((M, N), dtype=torch.float16, device=DEV)
+        call = lambda fd: lib.rocket_matmul_fp16(fd, M, K, N, R.ptr(a), R.ptr(b), R.ptr(out))  # noqa: E731
+    else:
+        H, n, d = 8, 1024, 128
+        a, b, v = h((H, 1, d), 8), h((H, n, d), 9), h((H, d, n), 10)
+        out = torch.empty((H, 1, d), dtype=torch.float16, device=DEV)
+        call = lambda fd: lib.rocket_flash_attn_fp16(fd, 1, n, d, d, H, H, d ** -0.5, 0.0, R.ptr(a), R.ptr(b), R.ptr(v),  # noqa: E731
+                                                     None, R.ptr(out))
+    torch.cuda.synchronize()
+    # eager first, on another handle, with slices and without: the kernels' one-time set-up
+    warm = lib.rocket_open()
+    _handle(lib, warm, stream)
+    assert call(warm) == 0
+    monkeypatch.setenv("ROCKET_HIP_SPLITK", "1")
+    assert call(warm) == 0
+    monkeypatch.delenv("ROCKET_HIP_SPLITK")
+    stream.synchronize()
+    eager = out.float().cpu().numpy()
+    fd = lib.rocket_open()
+    _handle(lib, fd, stream)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        rc = call(fd)
+    assert rc == 0
+    for _ in range(3):
+        with torch.cuda.stream(stream):
+            out.fill_(float("nan"))
+        stream.synchronize()
+        g.replay()
+        stream.synchronize()
+        got = out.float().cpu().numpy()
+        # fp32 sums in another order (and split outputs held in fp16): a rounding or two of fp16, of the
+        # largest value where terms cancel
+        assert np.max(np.abs(got - eager)) <= 2.0 ** -9 * np.max(np.abs(eager))
+    del g
+    lib.rocket_close(warm)
+    lib.rocket_close(fd)
