@@ -35,7 +35,7 @@ int rocket_quantize_rows_int8_fp16(int fd, int M, int K, const _Float16 *A, int8
 /* The resident group-wise products on fp32 activations: A is quantised per row into the
  * handle's arena by the pre-pass above, then the *_rowscale kernel runs with those codes and
  * scales — the same bits as rocket_quantize_rows_int8 followed by
- * rocket_matmul_int{8,4}_prepacked_gw_rowscale, in one call (two launches, the int8 codes
+ * rocket_matmul_int{8,4}_prepacked_gw_rowscale, in one call (two launches, or one that also quantises for few rows; the int8 codes
  * never leave the GPU). Same checks and return codes as the *_rowscale entry each mirrors. */
 int rocket_matmul_int8_prepacked_gw_f32in(rocket_i8_ctx *ctx, int M, int K, int N, const float *A,
                                           const float *b_scale, float *Cf, rocket_i8_weights *w);
@@ -74,7 +74,7 @@ int rocket_matmul_int8_prepacked_gw_grouped_glu_f16in(rocket_i8_ctx *ctx, int n,
  * other checks as the entry it mirrors. All calls on one GPU share the array: calls queued on
  * one stream are ordered and safe, calls that overlap on one GPU (several handles or streams
  * at once) race. While the handle's stream is being captured into a HIP graph the call only
- * records its two kernel launches (no wait, no memset, no copy) and returns 0; it returns -4
+ * records its kernel launches (no wait, no memset, no copy) and returns 0; it returns -4
  * if an earlier wait on the handle gave up, since draining it would end the capture. */
 int rocket_matmul_int4_prepacked_gw_f32in_noalloc(rocket_i4_ctx *ctx, int M, int K, int N, const float *A,
                                                    const float *b_scale, float *Cf, rocket_i4_weights *w);

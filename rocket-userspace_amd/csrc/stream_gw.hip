@@ -4,8 +4,8 @@
 // As in stream.hip the weights' bytes in flight bound the product, and here every output is one
 // fp32 chain over its groups in order, so a wave owns 16 columns and all of K: no partial
 // crosses waves and nothing but the prologue has a barrier. What keeps enough bytes in flight
-// with so few waves is LDS: a wave's weights go global -> LDS by DMA into a ring of its own, up
-// to 60 KB deep, each step's 16 rows x 64 bytes as one instruction (lane l: row l % 16, bytes
+// with so few waves is LDS: a wave's weights go global -> LDS by DMA into a ring of its own of
+// three 4 KB slots, each step's 16 rows x 64 bytes as one instruction (lane l: row l % 16, bytes
 // 16 (l / 16) .. + 16), and the ds_reads pick each group's bytes so that one MFMA covers
 // exactly one group's K or a part of it: with groups of 32 a 16x16x32 MFMA whose lane quarters
 // hold eight values each of the group. The activations' codes lie in LDS once a workgroup
@@ -69,7 +69,7 @@ __device__ __forceinline__ long lo64(i32x4 v) { return (long)(((unsigned long)(u
 // PK: K of an MFMA piece (32, 64 or, int4, 128), a divisor of the group; PPG: pieces a group (1 or
 // 2: whole groups a slot, so that a slot's body has no branch and its LDS reads, MFMAs and folds
 // overlap; 0: any number, counted). RS: a scale a row. QIN: 0 int8 codes in global memory, 1 / 2 fp32 / fp16 rows that each
-// workgroup quantises by k_quant_rows' formula (act(A) * A2 where A2 is given). W: waves.
+// workgroup quantises by k_quant_rows' formula (act(A) * A2 where A2 is given).
 template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT>
 __global__ __launch_bounds__(512, 2) void k_stream_gw(const GArgs a)
 {
