@@ -234,9 +234,10 @@ bool stream_takes(const Launch &L, int maxM)
     // A plain fp16 row keeps the bits that one chain over K gives it, whatever M, below K = 1024
     // (there the tiled kernels' chain is short, and k_small_f16 takes most such products).
     if (L.fmt_a == Fmt::F16 && (L.epi == Epi::F16 || L.epi == Epi::F32) && L.K < 1024) return false;
-    // one K range, results written once; operand rows are addressed with 32-bit byte offsets
+    // one K range, results written once; operand rows are addressed with 32-bit byte offsets (64 rows',
+    // the smallest tile's: longer rows are refused by the tiled kernels' own check)
     return maxM <= 16 && L.epi != Epi::GW && L.fmt_a != Fmt::I16 && !L.accum && L.kbeg == 0 && L.kend == L.K &&
-           maxM * row_bytes(L.fmt_a, L.K) < (1L << 31) && 16 * row_bytes(L.fmt_b, L.K) < (1L << 31);
+           64 * row_bytes(L.fmt_a, L.K) < (1L << 31) && 64 * row_bytes(L.fmt_b, L.K) < (1L << 31);
 }
 
 hipError_t stream_launch(const Launch &L, uint64_t *blocks)

@@ -387,6 +387,7 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
     const int sk = i4 ? 128 : 64;
     if (L.epi != Epi::GW || maxM > 16 || maxM < 1 || L.kt != L.group || L.fmt_a != Fmt::I8) return false;
     if (L.qa && (!L.rowscale || (L.qa == 2 && i4))) return false;
+    if (64 * row_bytes(L.fmt_a, L.K) >= (1L << 31)) return false;   // (refused by the tiled kernels' own check)
     for (int i = 0; i < L.nprob; i++)
         if (L.prob[i].dump) return false;
     g.np = 0;
