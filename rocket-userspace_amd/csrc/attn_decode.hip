@@ -55,7 +55,7 @@ struct RowArgs {
     int T, n_kv, dk, dv, gqa, n_head;
     float scale, softcap;
     int nsplit, cps;   // workgroups a KV head, chunks a workgroup
-    void *part;        // as attn.hip's: [split][head][T][dv] fp16, then [split][head][T] (max, sum)
+    float *part;       // [split][head][T][dv] outputs, then [split][head][T] (max, sum)
 };
 
 // Halves key .. key + 8 of a row of n (n >= 8), zeros past the row: the last eight are loaded
@@ -82,28 +82,32 @@ __device__ __forceinline__ i32x4 row8(const _Float16 *row, int key, int n)
 }
 
 // Merges the splits, one (head, token) row a workgroup: out = sum_s w_s On_s / sum_s w_s with
-// w_s = 2^(m_s - m) l_s, as attn.hip's k_fa_combine, for up to 64 splits. The splits spread over
+// w_s = 2^(m_s - m) l_s, for up to 64 splits. The outputs are fp32, as one workgroup without splits
+// holds them: caches from a few hundred keys on are split here, and a rounding of each split's output
+// to fp16 beside those of the probabilities and of the result would cost a fifth more error (192 to
+// 448 keys, heads of 256: 2.8e-4 of the result, with it 3.4e-4). The splits spread over
 // the workgroup's 256 threads (dv / 8 threads a split), whose sums add in LDS. (A merge by each KV
 // head's last workgroup instead of this launch, on an arrival counter, measured 15.5 against 11.1
 // us at 3000 keys: the counter's release and acquire write back and invalidate the XCD's L2, and
 // one workgroup walks all rows.)
-__global__ __launch_bounds__(256) void k_fa_merge(const void *__restrict__ part, _Float16 *__restrict__ O, long o_hs, long o_rs,
+__global__ __launch_bounds__(256) void k_fa_merge(const float *__restrict__ part, _Float16 *__restrict__ O, long o_hs, long o_rs,
                                                   int n_head, int T, int dv, int nsplit)
 {
     __shared__ float wt[64], sum[8 * 256];
     const int tid = threadIdx.x, row = blockIdx.x, h = row / T, t = row - h * T;
     const size_t rows = (size_t)n_head * T;
-    const _Float16 *po = static_cast<const _Float16 *>(part);
     const int dq = dv / 8, sg = tid / dq, d0 = (tid - sg * dq) * 8, ng = min(8, 256 / dq);   // dv <= 256: 8
-    f16x8 os[8];
+    f32x4 os[8][2];
     if (sg < ng)
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int s = sg + i * ng;
-            if (s < nsplit) os[i] = *reinterpret_cast<const f16x8 *>(po + ((size_t)s * rows + row) * dv + d0);
+            if (s < nsplit)
+#pragma unroll
+                for (int j = 0; j < 2; j++) os[i][j] = reinterpret_cast<const f32x4 *>(part + ((size_t)s * rows + row) * dv + d0)[j];
         }
     if (tid < 64) {
-        const f32x2 x = tid < nsplit ? reinterpret_cast<const f32x2 *>(po + (size_t)nsplit * rows * dv)[(size_t)tid * rows + row]
+        const f32x2 x = tid < nsplit ? reinterpret_cast<const f32x2 *>(part + (size_t)nsplit * rows * dv)[(size_t)tid * rows + row]
                                      : f32x2{-INFINITY, 0.f};
         float m = x[0];
 #pragma unroll
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(256) void k_fa_merge(const void *__restrict__ part,
             const int s = sg + i * ng;
             if (s < nsplit)
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[e] += wt[s] * (float)os[i][e];
+                for (int e = 0; e < 8; e++) acc[e] += wt[s] * os[i][e >> 2][e & 3];
         }
 #pragma unroll
         for (int e = 0; e < 8; e++) sum[sg * dv + d0 + e] = acc[e];
@@ -273,15 +277,14 @@ __global__ __launch_bounds__(kWaves * 64) void k_fa_rows(const RowArgs a)
         }
         const float inv = l > 0.f ? 1.f / l : 0.f;
         const int g = r / a.T, tt = r - g * a.T, h = hk * a.gqa + g;
-        f16x4 out;
-#pragma unroll
-        for (int e = 0; e < 4; e++) out[e] = (_Float16)(o[e] * inv);
         if (a.nsplit > 1) {
             const size_t row = ((size_t)zs * a.n_head + h) * a.T + tt;
-            *reinterpret_cast<f16x4 *>(static_cast<_Float16 *>(a.part) + row * a.dv + d0) = out;
-            if (d0 == 0)
-                reinterpret_cast<f32x2 *>(static_cast<_Float16 *>(a.part) + (size_t)a.nsplit * a.n_head * a.T * a.dv)[row] = f32x2{m, l};
+            *reinterpret_cast<f32x4 *>(a.part + row * a.dv + d0) = o * inv;
+            if (d0 == 0) reinterpret_cast<f32x2 *>(a.part + (size_t)a.nsplit * a.n_head * a.T * a.dv)[row] = f32x2{m, l};
         } else {
+            f16x4 out;
+#pragma unroll
+            for (int e = 0; e < 4; e++) out[e] = (_Float16)(o[e] * inv);
             *reinterpret_cast<f16x4 *>(a.O + (size_t)h * a.o_hs + (size_t)tt * a.o_rs + d0) = out;
         }
     }
@@ -337,7 +340,7 @@ size_t flash_attn_rows_ws(const FaLaunch &L)
 {
     int n, cps;
     split_of(L, &n, &cps);
-    return n > 1 ? (size_t)n * L.n_head * L.T * (L.dv * sizeof(_Float16) + 2 * sizeof(float)) : 0;
+    return n > 1 ? (size_t)n * L.n_head * L.T * (L.dv + 2) * sizeof(float) : 0;
 }
 
 hipError_t flash_attn_rows(const FaLaunch &L, hipStream_t s, uint64_t *blocks)

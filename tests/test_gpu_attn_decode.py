@@ -66,3 +66,26 @@ def test_attn_reads_no_other_row(lib, orc, fd, T, n):
     keep = np.arange(dv) != 17
     assert np.array_equal(out[:, :, keep], ref[:, :, keep])
     assert np.isposinf(orc.f16_bits_to_f32(np.ascontiguousarray(out[:, :, 17]))).all()
+
+
+@pytest.mark.parametrize("n,d,heads,kvh", [(192, 256, 16, 8), (448, 256, 16, 8), (448, 128, 32, 8), (3000, 256, 16, 8)])
+def test_attn_few_rows_error(lib, orc, fd, n, d, heads, kvh):
+    """The error against float64 is that of two roundings to fp16, the probabilities' and the result's,
+    also where the keys are split: a rounding is 2.07e-4 (2^-11 / sqrt(3), times 0.736, the root mean
+    square of 2^e / x over a log-uniform mantissa), two independent ones 2.93e-4, a third one (split
+    outputs in fp16) would make 3.59e-4. Bar: 2.93e-4 and 4 %, the sampling of 4096 results. The same
+    call again gives the same bits."""
+    print(f"attn error n={n} d={d} heads={heads}/{kvh}", flush=True)
+    Q, K, V = (orc.gen_normal(s, SEED + 30 + i).astype(np.float16) for i, s in enumerate(((heads, 1, d), (kvh, n, d), (kvh, d, n))))
+    out, again = np.empty((heads, 1, d), np.uint16), np.empty((heads, 1, d), np.uint16)
+    for o in (out, again):
+        assert lib.rocket_flash_attn_fp16(fd, 1, n, d, d, heads, kvh, d ** -0.5, 0.0, R.ptr(Q), R.ptr(K), R.ptr(V), None, R.ptr(o)) == 0
+    assert np.array_equal(out, again)
+    q, k, v = (x.astype(np.float64) for x in (Q, K, V))
+    k, v = np.repeat(k, heads // kvh, 0), np.repeat(v, heads // kvh, 0)
+    s = np.matmul(q, k.transpose(0, 2, 1)) * d ** -0.5
+    p = np.exp(s - s.max(2, keepdims=True))
+    want = np.matmul(p / p.sum(2, keepdims=True), v.transpose(0, 2, 1))
+    rel = np.linalg.norm(out.view(np.float16).astype(np.float64) - want) / np.linalg.norm(want)
+    print(f"  rel {rel:.3e}", flush=True)
+    assert rel <= 3.05e-4
