@@ -34,6 +34,7 @@ struct F16Product {
         L.kbeg = 0;
         L.kend = K;
         L.nprob = 1;
+        L.free_sums = 1;
         L.prob[0].M = M;
         ws = gemm_ws_bytes(L);
     }

@@ -67,6 +67,9 @@ struct Launch {
     int act = 0;              // GLU / ACT, or qa with A2: kActSilu or kActGelu
     int qa = 0;               // GW, rowscale: A holds fp32 (1) or fp16 (2) rows, quantised per row in the kernel
                               // (quant_rows' formula; only where gemm_quantises says so)
+    int free_sums = 0;        // plain fp16: 1, K may be summed in any slices (a block's own product); 0, the slices
+                              // depend on the tiles' plan for M > 128 alone, so that a row's bits do not depend
+                              // on the launch's other problems, nor, up to 128 rows, on M
     int f16out = 0;           // GW: C holds fp16 (each fp32 result rounded once) instead of fp32
     int kt = 0;               // GW: int32 partial period, divides group (== group normally)
     int nprob = 0;

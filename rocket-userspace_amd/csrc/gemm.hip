@@ -438,8 +438,8 @@ Choice choose(Fmt fa, Fmt fb, Epi epi, int maxM, int kspan, long outs, bool accu
     return {64, 64, 1};
 }
 
-// Products of fp16 / fp32 operands whose tiles leave the GPU waiting for one workgroup's chain of
-// stages: K in slices of smaller tiles, by estimated time. A stage takes its latency, or, with n
+// Products of fp32 operands (and fp16 ones whose sums are free, Launch::free_sums) whose tiles leave
+// the GPU waiting for one workgroup's chain of stages: K in slices of smaller tiles, by estimated time. A stage takes its latency, or, with n
 // workgroups on a CU, the n stages' operand bytes at 58 KB / us or their MFMAs, whichever is
 // longest; slices add a launch and their planes' bytes. The constants are fits to 40 products of 24
 // to 1024 rows, every tile and slice count timed (the estimate's choice took at most 1.2 times the
@@ -480,20 +480,20 @@ double plan_time(const FloatMath &m, const StageFit &f, int M, int K, int N, int
 }
 
 // The estimate's choice for one product, where it takes at most 0.85 of the time of `base` (the choice
-// of choose() on unconverted operands, so that converting them first changes no slicing). A plain
-// fp16 row keeps the bits that one chain over K gives it, whatever M and N, up to K = 2048.
-bool choose_slices(Fmt fa, int M, int K, int N, const Choice &base, Choice *out)
+// of choose() on unconverted operands, so that converting them first changes no slicing). With
+// `keep` the slices stay the base's and the tile alone is chosen: the same bits.
+bool choose_slices(Fmt fa, int M, int K, int N, const Choice &base, bool keep, Choice *out)
 {
     if (base.bn == 256) return false;
     const FloatMath m = float_math(fa);
     const char *env = getenv("ROCKET_HIP_SPLITK");
-    const int cap = env ? splitk_cap() : 8, most = fa == Fmt::F16 && K <= 2048 ? 1 : cap;
+    const int least = keep ? base.splitk : 1, most = keep ? base.splitk : env ? splitk_cap() : 8;
     double now = 0, best = 0;
     for (int i = 0; i < m.n; i++) {
         const StageFit &f = m.fit[i];
         if (f.bm == base.bm && f.bn == base.bn) now = plan_time(m, f, M, K, N, base.splitk);
-        for (int z = 1; z <= most; z *= 2) {
-            if (z > 1 && K / z < 256) break;
+        for (int z = least; z <= most; z *= 2) {
+            if (z > 1 && !keep && K / z < 256) break;
             const double t = plan_time(m, f, M, K, N, z);
             if (best == 0 || t < best) {
                 best = t;
@@ -534,7 +534,7 @@ Plan plan_of(const Launch &L, int maxM, bool allow_split)
         const Fmt raw = L.fmt_a == Fmt::BF16 ? Fmt::F32BF16 : L.fmt_a == Fmt::BF16X2 ? Fmt::F32TF32 : L.fmt_a;
         const Choice base = choose(raw, raw, L.epi, maxM, kspan, outs, split_ok, tiles);
         Choice x;
-        if (choose_slices(L.fmt_a, maxM, L.K, L.N, base, &x)) c = x;
+        if (choose_slices(L.fmt_a, maxM, L.K, L.N, base, one_chain(L), &x)) c = x;
     }
     Plan p;
     p.bm = c.bm;

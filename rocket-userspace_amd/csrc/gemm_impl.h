@@ -1881,6 +1881,9 @@ hipError_t dispatch_bf16(int bm, int bn, const Launch &L, const KArgs &ka, int b
 // HBM bytes of one operand row of K elements.
 long row_bytes(Fmt f, int K);
 
+// A plain fp16 product whose rows keep the bits of one chain over K.
+inline bool one_chain(const Launch &L) { return L.fmt_a == Fmt::F16 && (L.epi == Epi::F16 || L.epi == Epi::F32) && !L.free_sums; }
+
 // Products of at most 16 rows (stream.hip): whether the launch takes the weight-streaming
 // kernel, and its launch.
 bool stream_takes(const Launch &L, int maxM);
