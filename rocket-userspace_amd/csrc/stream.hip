@@ -1,4 +1,4 @@
-// stream.hip — products of at most 16 rows (decode batches): the weight-streaming kernel.
+// stream.hip — products of at most 16 rows (decode batches): the weight-streaming kernels.
 //
 // With so few activation rows a product reads every weight once and does little with it: what
 // bounds it is how many bytes of B are in flight. The tiled kernels (gemm_impl.h) walk K in LDS
@@ -9,11 +9,10 @@
 // every workgroup) as the first, one set of steps in flight while the other's MFMAs run. The
 // waves' sums meet in LDS once, at the end, added in wave order. fp32 operands are truncated or
 // split in registers, so no conversion pass runs first. The K slices depend on the formats and
-// K alone: a row's bits do not depend on N, on M up to 16, or on the launch's other problems.
+// K alone: a row's bits do not depend on N, on M up to 16, or on the launch's other problems. Plain
+// fp16 products, whose rows have the tiled kernels' bits, take k_chain instead: one wave, all of K.
 //
 // Measured (three sets of operands in turn; tiled kernels before, this kernel after):
-//   fp16     4 x  4096 x  4096   21.5 ->  7.9 us   (4.2 TB/s)
-//   fp16    16 x  3840 x 15360   33.5 -> 31.3 us
 //   int8     4 x  4096 x  4096    8.0 ->  5.8 us
 //   bf16     4 x  4096 x  4096   29.1 -> 13.1 us   (fp32 operands, 5.1 TB/s)
 //   tf32     4 x  4096 x  4096   46.8 -> 13.4 us
@@ -194,6 +193,110 @@ __global__ __launch_bounds__(KS * 64, 4) void k_stream(const SArgs a)
     }
 }
 
+// Plain fp16 products: one chain over K in order, so that a row has the same bits among 16 rows, among
+// 20 or 128 (tiles, whose 32x32x16 MFMAs sum 32 values of K to the same bits as one 16x16x32), and in
+// a batch. A wave owns 16 NB columns, MB blocks of 16 rows and all of K; lane l loads row (or column)
+// l % 16, halves 8 (l / 16) .. + 8 of a step of 32. What bounds it is the loads in flight, of which a wave
+// can count 63: SETS sets of four steps' operands, each set loaded again as soon as its MFMAs are issued.
+// Measured (start of this kernel: K in eight slices, k_stream; tiles): 4 x 4096 x 4096 9.9 us (8.0;
+// 21.4), 4 x 2048 x 4096 6.3 (5.9; 12.7), 4 x 4096 x 16384 23.9 (30.3; 31.8), 20 x 4096 x 4096 13.5 (tiles 22.1).
+constexpr int kChainSteps = 4;
+
+template <int... I, class F> __device__ __forceinline__ void each(std::integer_sequence<int, I...>, F &&f)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int MB, int NB, int SETS, bool F16OUT>
+__global__ __launch_bounds__(64) void k_chain(const SArgs a)
+{
+    const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
+    const int p = blockIdx.y, M = a.M[p], n0 = (int)blockIdx.x * 16 * NB;
+    if (M == 0) return;
+    const Rsrc ra = rsrc(a.A[p], (uint32_t)M * a.lda);   // rows past M and columns past N lie past the ranges: zeros
+    const Rsrc rb = rsrc(static_cast<const char *>(a.B[p]) + (size_t)n0 * a.ldb, (uint32_t)min(16 * NB, a.N - n0) * a.ldb);
+    const uint32_t o = (uint32_t)r * a.lda + (uint32_t)q * 16u, blk = 16u * a.lda;   // lda == ldb
+    i32x4 fa[SETS][kChainSteps][MB], fb[SETS][kChainSteps][NB];
+    f32x4 acc[MB][NB];
+#pragma unroll
+    for (int x = 0; x < MB; x++)
+#pragma unroll
+        for (int y = 0; y < NB; y++) acc[x][y] = f32x4{};
+    auto load = [&](auto SET, int c) __attribute__((always_inline)) {
+        constexpr int t = decltype(SET)::value;
+#pragma unroll
+        for (int i = 0; i < kChainSteps; i++) {
+            const int st = c * kChainSteps + i;   // past K: zeros, whose MFMAs add nothing
+            const uint32_t off = st < a.nsteps ? o + (uint32_t)st * 64u : kOOB;
+#pragma unroll
+            for (int y = 0; y < NB; y++) fb[t][i][y] = ld16(rb, off + y * blk);
+#pragma unroll
+            for (int x = 0; x < MB; x++) fa[t][i][x] = ld16(ra, off + x * blk);
+        }
+    };
+    auto mma = [&](auto SET) __attribute__((always_inline)) {
+        constexpr int t = decltype(SET)::value;
+#pragma unroll
+        for (int i = 0; i < kChainSteps; i++)
+#pragma unroll
+            for (int y = 0; y < NB; y++)
+#pragma unroll
+                for (int x = 0; x < MB; x++)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, fa[t][i][x]), __builtin_bit_cast(f16x8, fb[t][i][y]),
+                                                                       acc[x][y], 0, 0, 0);
+    };
+    const int nch = (a.nsteps + kChainSteps - 1) / kChainSteps;
+    using Sets = std::make_integer_sequence<int, SETS>;
+    each(Sets{}, [&](auto S) __attribute__((always_inline)) { load(S, decltype(S)::value); });
+    for (int c = 0; c < nch; c += SETS)
+        each(Sets{}, [&](auto S) __attribute__((always_inline)) {
+            constexpr int i = decltype(S)::value;
+            if (c + i < nch) {
+                mma(S);
+                if (c + i + SETS < nch) load(S, c + i + SETS);
+            }
+        });
+#pragma unroll
+    for (int y = 0; y < NB; y++) {
+        const int n = n0 + 16 * y + r;
+        if (n >= a.N) continue;
+#pragma unroll
+        for (int x = 0; x < MB; x++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int m = 16 * x + 4 * q + e;
+                if (m >= M) continue;
+                const size_t at = (size_t)m * a.N + n;
+                if constexpr (F16OUT) static_cast<_Float16 *>(a.C[p])[at] = (_Float16)acc[x][y][e];
+                else static_cast<float *>(a.C[p])[at] = acc[x][y][e];
+            }
+    }
+}
+
+hipError_t launch_chain(SArgs &a, const Launch &L, uint64_t *blocks)
+{
+    a.nsteps = L.K / 32;
+    int maxM = 0;
+    for (int i = 0; i < L.nprob; i++) maxM = std::max(maxM, L.prob[i].M);
+    auto go = [&](auto MB, auto NB, auto SETS) {
+        constexpr int mb = decltype(MB)::value, nb = decltype(NB)::value, sets = decltype(SETS)::value;
+        const dim3 grid((unsigned)((a.N + 16 * nb - 1) / (16 * nb)), (unsigned)L.nprob);
+        *blocks = (uint64_t)grid.x * grid.y;
+        if (L.epi == Epi::F16) hipLaunchKernelGGL((k_chain<mb, nb, sets, true>), grid, dim3(64), 0, L.stream, a);
+        else hipLaunchKernelGGL((k_chain<mb, nb, sets, false>), grid, dim3(64), 0, L.stream, a);
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I5 = std::integral_constant<int, 5>;
+    using I7 = std::integral_constant<int, 7>;
+    // two column blocks a wave share the rows' fragments where the columns still give a CU two waves
+    // (16 x 3072 x 16384 23.6 -> 19.8 us; 16 x 4096 x 8192 17.2 and 18.5)
+    if (maxM > 16) go(I2{}, I1{}, I5{});
+    else if (maxM > 4 && a.N >= 16384) go(I1{}, I2{}, I5{});
+    else go(I1{}, I1{}, I7{});
+    return hipGetLastError();
+}
+
 template <Fmt FA, Fmt FB, int KS> hipError_t launch_ks(SArgs &a, const Launch &L, uint64_t *blocks)
 {
     a.per = (a.nsteps + KS - 1) / KS;
@@ -231,12 +334,15 @@ template <Fmt FA, Fmt FB> hipError_t launch_fmt(SArgs &a, const Launch &L, uint6
 
 bool stream_takes(const Launch &L, int maxM)
 {
-    // A plain fp16 row keeps the bits that one chain over K gives it, whatever M, below K = 1024
-    // (there the tiled kernels' chain is short, and k_small_f16 takes most such products).
-    if (L.fmt_a == Fmt::F16 && (L.epi == Epi::F16 || L.epi == Epi::F32) && L.K < 1024) return false;
+    const bool plain = L.fmt_a == Fmt::F16 && (L.epi == Epi::F16 || L.epi == Epi::F32);
+    // Below K = 1024 a plain fp16 product's chain is short, and k_small_f16 takes most such products.
+    if (plain && L.K < 1024) return false;
+    // One chain a wave serves 32 rows too, until the columns give the tiles half the CUs (20 x 4096 x 4096
+    // 13.5 us, tiles 22.1; 32 rows 15.4 and 22.3; at 8192 columns 32 x 2048 14.1 and 13.5).
+    const int most = one_chain(L) && (long)L.nprob * L.N < 8192 ? 32 : 16;
     // one K range, results written once; operand rows are addressed with 32-bit byte offsets (64 rows',
     // the smallest tile's: longer rows are refused by the tiled kernels' own check)
-    return maxM <= 16 && L.epi != Epi::GW && L.fmt_a != Fmt::I16 && !L.accum && L.kbeg == 0 && L.kend == L.K &&
+    return maxM <= most && L.epi != Epi::GW && L.fmt_a != Fmt::I16 && !L.accum && L.kbeg == 0 && L.kend == L.K &&
            64 * row_bytes(L.fmt_a, L.K) < (1L << 31) && 64 * row_bytes(L.fmt_b, L.K) < (1L << 31);
 }
 
@@ -259,6 +365,7 @@ hipError_t stream_launch(const Launch &L, uint64_t *blocks)
         a.C[i] = P.C;
     }
     const Fmt fa = L.fmt_a, fb = L.fmt_b;
+    if (one_chain(L)) return launch_chain(a, L, blocks);
     if (fa == Fmt::F16) return launch_fmt<Fmt::F16, Fmt::F16>(a, L, blocks);
     if (fa == Fmt::I8 && fb == Fmt::I8) return launch_fmt<Fmt::I8, Fmt::I8>(a, L, blocks);
     if (fa == Fmt::I8 && fb == Fmt::I4P) return launch_fmt<Fmt::I8, Fmt::I4P>(a, L, blocks);

@@ -116,3 +116,26 @@ def test_stream_under_capture(lib, orc):
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
     lib.rocket_close(fd)
+
+
+@pytest.mark.parametrize("K,N", [(K, N) for K in (992, 1024, 1056, 1472, 2048, 4096, 8224) for N in (16, 208)] + [(1056, 16400)])
+def test_fp16_rows_have_the_bits_of_larger_calls(lib, orc, fd, K, N):
+    """A plain fp16 row's sum is one chain over K: the rows of a product of 100 rows (tiles) against
+    calls of its first 1, 4, 16, 20, 32 (one wave a column block) and 64 rows, with fp32 results (every
+    bit of the sum) and fp16 ones; K of whole sets of loads and of a part of one, and fewer sets than a
+    wave keeps in flight."""
+    print(f"fp16 rows K={K} N={N}", flush=True)
+    M = 100
+    # magnitudes over 2^16, so that the order of the sums shows
+    A = orc.f32_to_f16_bits(orc.gen_normal((M, K), SEED + 50) * np.exp2(orc.gen_uniform((M, K), SEED + 52, -8.0, 8.0)))
+    B = orc.f32_to_f16_bits(orc.gen_normal((N, K), SEED + 51, 0, 0.02))
+    big = np.empty((M, N), np.float32)
+    assert lib.rocket_matmul_fp16_f32out(fd, M, K, N, R.ptr(A), R.ptr(B), R.ptr(big)) == 0
+    assert orc.norm_err(big, orc.matmul_fp16_f32out(A, B)) < 1e-5
+    for m in (1, 4, 16, 20, 32, 64):
+        out, h = np.full((m, N), np.nan, np.float32), np.empty((m, N), np.uint16)
+        Am = np.ascontiguousarray(A[:m])
+        assert lib.rocket_matmul_fp16_f32out(fd, m, K, N, R.ptr(Am), R.ptr(B), R.ptr(out)) == 0
+        assert np.array_equal(out, big[:m]), m
+        assert lib.rocket_matmul_fp16(fd, m, K, N, R.ptr(Am), R.ptr(B), R.ptr(h)) == 0
+        assert np.array_equal(h, orc.f32_to_f16_bits(big[:m])), m
