@@ -60,7 +60,9 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     if (pad) c.want_scratch(h16((size_t)n_kv_heads * dv * n_kvp));
     const bool pad_m = pad && mask && (size_t)T * n_kvp < ((size_t)1 << 30);   // (32-bit offsets into it)
     if (pad_m) c.want_scratch(h16((size_t)T * n_kvp));
-    const size_t ws = c.want_optional(flash_attn_ws_bytes(f));
+    // (a graph of a call over a short cache holds no scratch: unsplit it takes at most a few us more,
+    // while a long one would run many times as long)
+    const size_t ws = c.want_optional(flash_attn_ws_bytes(f), n_kv >= 512);
     if (int rc = c.begin()) return rc;
     f.ws = ws ? static_cast<float *>(c.scratch(ws)) : nullptr;
     f.ws_bytes = f.ws ? ws : 0;

@@ -223,14 +223,17 @@ void Call::want(const void *p, size_t bytes)
     if (!direct_(p)) need_ += round_(bytes);
 }
 
-size_t Call::want_optional(size_t bytes)
+bool Call::capturing_()
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(h_->stream, &cap) != hipSuccess) (void)hipGetLastError();
+    return cap != hipStreamCaptureStatusNone;
+}
+
+size_t Call::want_optional(size_t bytes, bool worth)
 {
     if (bytes == 0) return 0;
-    if (need_ + round_(bytes) > h_->arena_cap) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(h_->stream, &cap) != hipSuccess) (void)hipGetLastError();
-        if (cap != hipStreamCaptureStatusNone) return 0;
-    }
+    if ((need_ + round_(bytes) > h_->arena_cap || (need_ == 0 && !worth)) && capturing_()) return 0;
     want_scratch(bytes);
     return bytes;
 }
@@ -244,7 +247,9 @@ int Call::begin()
     }
     if (need_ > h_->arena_cap) {
         if (hipStreamSynchronize(h_->stream) != hipSuccess) { (void)hipGetLastError(); return err_ = ROCKET_E_DEVICE; }
-        dev_free(h_->arena);
+        if (h_->arena_held) h_->retired.push_back(h_->arena);
+        else dev_free(h_->arena);
+        h_->arena_held = false;
         h_->arena = nullptr;
         h_->arena_cap = 0;
         const size_t cap = need_ + need_ / 4;
@@ -252,6 +257,7 @@ int Call::begin()
         if (!h_->arena) return err_ = ROCKET_E_NOMEM;
         h_->arena_cap = cap;
     }
+    if (need_ > 0 && !h_->arena_held) h_->arena_held = capturing_();
     return ROCKET_OK;
 }
 
@@ -422,6 +428,8 @@ void rocket_close(int fd)
         if (hipSetDevice(h->device) == hipSuccess) {
             (void)hipStreamSynchronize(h->stream);
             dev_free(h->arena);
+            for (void *p : h->retired) dev_free(p);
+            h->retired.clear();
             h->arena = nullptr;
             h->arena_cap = 0;
             if (h->pin) (void)hipHostFree(h->pin);

@@ -27,6 +27,8 @@ struct Handle {
     bool dirty = false;            // a wait timed out: drain before reusing buffers
     bool closed = false;           // rocket_close ran: buffers released, no further work
     void *arena = nullptr;  size_t arena_cap = 0;   // device staging
+    bool arena_held = false;                        // a captured call's graph holds the arena's address
+    std::vector<void *> retired;                    // outgrown arenas that graphs hold, until the close
     void *pin = nullptr;    size_t pin_cap = 0;     // pinned host staging for results
     std::mutex mu;
 };
@@ -58,11 +60,15 @@ public:
     // Reserve arena space before in()/out(): sum of every host operand's bytes.
     void want(const void *p, size_t bytes);
     void want_scratch(size_t bytes) { need_ += round_(bytes); }
-    // Scratch that the launch can do without (K slices' planes): `bytes`, reserved, or 0 where the
-    // arena would have to grow while the handle's stream is being captured, which allows no
-    // allocation. The last of the reservations.
-    size_t want_optional(size_t bytes);
-    int  begin();                          // grows the arena if needed
+    // Scratch that the launch can do without (K slices' planes, key splits' partials): `bytes`,
+    // reserved, or 0. While the handle's stream is being captured that is 0 where the arena would have
+    // to grow, which a capture does not allow, and where the call has no other scratch, unless it is
+    // `worth` it: a graph that holds scratch of the handle must not run beside its other work. The
+    // last of the reservations.
+    size_t want_optional(size_t bytes, bool worth);
+    // Grows the arena if needed. One that a captured call has used is kept until the handle closes:
+    // the graph replays on it (each at least 1.25 times the last, so all of them at most 5 times it).
+    int  begin();
     void *in(const void *p, size_t bytes);  // device view of an input
     void *out(void *p, size_t bytes);       // device view of an output
     void *scratch(size_t bytes);            // arena scratch (not copied)
@@ -75,6 +81,7 @@ public:
 private:
     static size_t round_(size_t b) { return (b + 255) & ~(size_t)255; }
     bool direct_(const void *p) const;
+    bool capturing_();
     int finish_();
     // ROCKET_MM_PROFILE: host milliseconds of this call's phases (staging copies and arena
     // growth, kernel enqueue, the bounded wait, result copy-out), added to the process totals

@@ -189,7 +189,8 @@ int run(int fd, const Req &r)
             Lp.kend = (r.kchunk > 0 && r.K > r.kchunk) ? r.kchunk : r.K;
             ws = std::max(ws, gemm_ws_bytes(Lp));
         }
-        ws = c.want_optional(ws);
+        // (bf16 / tf32 products of few columns, which convert no rows ahead, hold no scratch in a graph)
+        ws = c.want_optional(ws, r.fa == Fmt::F16 || r.N >= 256);
     }
     if (int rc = c.begin()) return rc;
     int32_t *wsp = ws ? static_cast<int32_t *>(c.scratch(ws)) : nullptr;

@@ -1,0 +1,108 @@
+// arena_check.cpp — what the library's calls do with a handle's scratch, on the fake runtime of
+// fake_hip.h: which kernels a call launches where the arena may not grow (a captured stream), what a
+// captured call's graph may still replay on after the arena has grown, and what is freed when the
+// handle closes. Built and run by tests/test_arena.py. Exit status 0 when every check passes.
+#include "fake_hip.h"
+
+#include <stdio.h>
+
+#include "rocket_attn.h"
+#include "rocket_ffn.h"
+#include "rocket_hip.h"
+#include "rocket_matmul.h"
+#include "rocket_npu.h"
+
+static int g_fail = 0;
+#define CHECK(c)                                                                                       \
+    do {                                                                                               \
+        if (!(c)) {                                                                                    \
+            fprintf(stderr, "arena_check: %s:%d: CHECK(%s) failed\n", __FILE__, __LINE__, #c);         \
+            g_fail++;                                                                                  \
+        }                                                                                              \
+    } while (0)
+
+static int open_async()
+{
+    const int fd = rocket_open();
+    CHECK(fd >= 0);
+    CHECK(rocket_hip_set_mode(fd, ROCKET_HIP_ASYNC | ROCKET_HIP_DEVICE_OPERANDS) == 0);
+    fake::st().launches.clear();
+    return fd;
+}
+
+// Operands: addresses that no kernel reads here.
+static float *const X = reinterpret_cast<float *>(0x100000);
+static float *const W = reinterpret_cast<float *>(0x10000000);
+static float *const Y = reinterpret_cast<float *>(0x20000000);
+static _Float16 *h(float *p) { return reinterpret_cast<_Float16 *>(p); }
+
+static int bf16(int fd, int M, int K, int N) { return rocket_matmul_bf16(fd, M, K, N, X, W, Y); }
+static int fp16(int fd, int M, int K, int N) { return rocket_matmul_fp16(fd, M, K, N, h(X), h(W), h(Y)); }
+static int attn(int fd, int T, int n)
+{
+    return rocket_flash_attn_fp16(fd, T, n, 128, 128, 8, 8, 0.1f, 0.f, h(X), h(W), h(W), nullptr, h(Y));
+}
+
+// Recorded while the stream is captured: the names of its launches.
+template <class F> static std::vector<std::string> captured(F call, int want_rc = 0)
+{
+    auto &f = fake::st();
+    f.launches.clear();
+    f.capturing = true;
+    const int syncs = f.syncs;
+    const int rc = call();
+    f.capturing = false;
+    CHECK(rc == want_rc);
+    if (rc == 0) CHECK(f.syncs == syncs);
+    return f.launches;
+}
+
+// A captured call's arena outlives its growth, and goes with the handle.
+static void arena_kept_for_graphs()
+{
+    auto &f = fake::st();
+    const int live0 = (int)f.live.size();
+    const int fd = open_async();
+    CHECK(attn(fd, 1, 4096) == 0);                       // eager: the arena
+    CHECK((int)f.live.size() == live0 + 1);
+    CHECK(captured([&] { return attn(fd, 1, 4096); }).size() == 2);   // keys split, and the merge
+    const int frees = f.frees;
+    CHECK(rocket_ffn_fp16(fd, 512, 1024, 8192, h(X), h(W), h(W), h(W), ROCKET_ACTIVATION_SILU, h(Y)) == 0);   // a larger arena
+    CHECK(f.frees == frees && (int)f.live.size() == live0 + 2);
+    // one that no graph holds is freed when it grows
+    CHECK(rocket_ffn_fp16(fd, 512, 1024, 16384, h(X), h(W), h(W), h(W), ROCKET_ACTIVATION_SILU, h(Y)) == 0);
+    CHECK(f.frees == frees + 1 && (int)f.live.size() == live0 + 2);
+    rocket_close(fd);
+    CHECK((int)f.live.size() == live0);
+}
+
+// Calls that can do without scratch hold none in a graph, on a handle that has some.
+static void small_calls_hold_no_scratch()
+{
+    const int fd = open_async();
+    CHECK(rocket_ffn_fp16(fd, 512, 1024, 8192, h(X), h(W), h(W), h(W), ROCKET_ACTIVATION_SILU, h(Y)) == 0);
+    fake::st().launches.clear();
+    CHECK(bf16(fd, 300, 15360, 96) == 0);
+    CHECK(fake::count("k_sum_slices") == 1);             // eager: K slices
+    CHECK(captured([&] { return bf16(fd, 300, 15360, 96); }).size() == 1);
+    CHECK(captured([&] { return attn(fd, 1, 448); }).size() == 1);
+    CHECK(captured([&] { return attn(fd, 1, 1000); }).size() == 2);
+    CHECK(captured([&] { return fp16(fd, 64, 4096, 4096); }).size() == 1);
+    CHECK(captured([&] { return fp16(fd, 4, 4096, 4096); }).size() == 1);
+    // a call that converts its rows ahead holds scratch anyway
+    captured([&] { return bf16(fd, 128, 8192, 512); });
+    CHECK(fake::count("k_cvt") == 1 && fake::count("k_sum_slices") == 1);
+    rocket_close(fd);
+}
+
+int main()
+{
+    arena_kept_for_graphs();
+    small_calls_hold_no_scratch();
+    if (g_fail) {
+        fprintf(stderr, "arena_check: %d check(s) failed\n", g_fail);
+        return 1;
+    }
+    printf("arena_check: all checks passed\n");
+    return 0;
+}
