@@ -38,7 +38,7 @@ struct F16Product {
         L.prob[0].M = M;
         ws = gemm_ws_bytes(L);
     }
-    void want_ws(Call &c) const { c.want_scratch(ws); }
+    void want_ws(Call &c) { ws = c.want_optional(ws, true); }   // the last of the reservations
     int run(Call &c, const void *A, const void *W, void *out)
     {
         L.prob[0] = Problem{L.prob[0].M, A, W, out, nullptr, nullptr, nullptr};

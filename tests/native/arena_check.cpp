@@ -95,10 +95,32 @@ static void small_calls_hold_no_scratch()
     rocket_close(fd);
 }
 
+// A block's second product runs without its K slices where the arena holds the hidden rows alone.
+static void blocks_on_a_small_arena()
+{
+    const int M = 64, H = 3840, I = 15360;
+    auto ffn = [&](int fd) { return rocket_ffn_fp16(fd, M, H, I, h(X), h(W), h(W), h(W), ROCKET_ACTIVATION_SILU, h(Y)); };
+    auto mlp = [&](int fd) { return rocket_mlp_fp16_fused(fd, M, H, I, H, h(X), h(W), nullptr, h(W), ROCKET_ACTIVATION_GELU, h(Y)); };
+    for (int which = 0; which < 2; which++) {
+        auto call = [&](int fd) { return which ? mlp(fd) : ffn(fd); };
+        const int fd = open_async();
+        setenv("ROCKET_HIP_SPLITK", "1", 1);
+        CHECK(call(fd) == 0);
+        unsetenv("ROCKET_HIP_SPLITK");
+        CHECK(captured([&] { return call(fd); }).size() == 2);
+        fake::st().launches.clear();
+        CHECK(call(fd) == 0);
+        CHECK(fake::count("k_sum_slices") == 1);                  // eager: the arena grows
+        CHECK(captured([&] { return call(fd); }).size() == 3);    // and then holds the slices too
+        rocket_close(fd);
+    }
+}
+
 int main()
 {
     arena_kept_for_graphs();
     small_calls_hold_no_scratch();
+    blocks_on_a_small_arena();
     if (g_fail) {
         fprintf(stderr, "arena_check: %d check(s) failed\n", g_fail);
         return 1;
