@@ -58,33 +58,37 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     if (mask) c.want(mask, h16(nm));
     c.want(out, h16(no));
     if (pad) c.want_scratch(h16((size_t)n_kv_heads * dv * n_kvp));
-    const bool pad_m = pad && mask && (size_t)T * n_kvp < ((size_t)1 << 30);   // (32-bit offsets into it)
-    if (pad_m) c.want_scratch(h16((size_t)T * n_kvp));
+    // (32-bit offsets into the padded mask)
+    const size_t mb = pad && mask && (size_t)T * n_kvp < ((size_t)1 << 30) ? c.want_optional(h16((size_t)T * n_kvp), true) : 0;
     // (a graph of a call over a short cache holds no scratch: unsplit it takes at most a few us more,
     // while a long one would run many times as long)
     const size_t ws = c.want_optional(flash_attn_ws_bytes(f), n_kv >= 512);
     if (int rc = c.begin()) return rc;
-    f.ws = ws ? static_cast<float *>(c.scratch(ws)) : nullptr;
+    f.ws = static_cast<float *>(c.optional(ws));
     f.ws_bytes = f.ws ? ws : 0;
     f.Q = static_cast<const _Float16 *>(c.in(Q, h16(nq)));
     f.K = static_cast<const _Float16 *>(c.in(K, h16(nk)));
     const _Float16 *dV = static_cast<const _Float16 *>(c.in(V, h16(nv)));
     f.mask = mask ? static_cast<const _Float16 *>(c.in(mask, h16(nm))) : nullptr;
+    f.m_rs = n_kv;
     f.O = static_cast<_Float16 *>(c.out(out, h16(no)));
     if (!f.Q || !f.K || !dV || (mask && !f.mask) || !f.O) return c.finish();
     if (pad) {
         _Float16 *vp = static_cast<_Float16 *>(c.scratch(h16((size_t)n_kv_heads * dv * n_kvp)));
-        _Float16 *mp = pad_m ? static_cast<_Float16 *>(c.scratch(h16((size_t)T * n_kvp))) : nullptr;
-        if (!vp || (pad_m && !mp)) return c.finish();
+        _Float16 *mp = static_cast<_Float16 *>(c.optional(mb));
+        if (!vp) return c.finish();
         uint64_t pb = 0;
-        if (pad_cols_f16(dV, vp, (long)n_kv_heads * dv, f.mask, mp, pad_m ? T : 0, n_kv, n_kvp, c.stream(), &pb) != hipSuccess) {
+        if (pad_cols_f16(dV, vp, (long)n_kv_heads * dv, f.mask, mp, mp ? T : 0, n_kv, n_kvp, c.stream(), &pb) != hipSuccess) {
             (void)hipGetLastError();
             ROCKET_LOGE("%s: V pad launch rejected\n", who);
             (void)c.finish();
             return ROCKET_E_DEVICE;
         }
         count_launch(pb);
-        if (pad_m) f.mask = mp;
+        if (mp) {
+            f.mask = mp;
+            f.m_rs = n_kvp;
+        }
         dV = vp;
     }
     f.Vt = dV;
@@ -92,7 +96,6 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     f.k_hs = (long)n_kv * dk; f.k_rs = dk;
     f.v_hs = (long)dv * n_kvp; f.v_rs = n_kvp;
     f.o_hs = (long)T * dv; f.o_rs = dv;
-    f.m_rs = pad_m ? n_kvp : n_kv;
     uint64_t blocks = 0;
     if (flash_attn(f, c.stream(), &blocks) != hipSuccess) {
         (void)hipGetLastError();

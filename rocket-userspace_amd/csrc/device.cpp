@@ -233,8 +233,8 @@ bool Call::capturing_()
 size_t Call::want_optional(size_t bytes, bool worth)
 {
     if (bytes == 0) return 0;
-    if ((need_ + round_(bytes) > h_->arena_cap || (need_ == 0 && !worth)) && capturing_()) return 0;
-    want_scratch(bytes);
+    if ((need_ + opt_ + round_(bytes) > h_->arena_cap || (need_ == 0 && !worth)) && capturing_()) return 0;
+    opt_ += round_(bytes);
     return bytes;
 }
 
@@ -245,19 +245,26 @@ int Call::begin()
         if (hipStreamSynchronize(h_->stream) != hipSuccess) { (void)hipGetLastError(); return err_ = ROCKET_E_DEVICE; }
         h_->dirty = false;
     }
-    if (need_ > h_->arena_cap) {
+    if (need_ + opt_ > h_->arena_cap) {
         if (hipStreamSynchronize(h_->stream) != hipSuccess) { (void)hipGetLastError(); return err_ = ROCKET_E_DEVICE; }
         if (h_->arena_held) h_->retired.push_back(h_->arena);
         else dev_free(h_->arena);
         h_->arena_held = false;
         h_->arena = nullptr;
         h_->arena_cap = 0;
-        const size_t cap = need_ + need_ / 4;
-        h_->arena = dev_alloc(cap, who_);
-        if (!h_->arena) return err_ = ROCKET_E_NOMEM;
+        size_t cap = need_ + opt_ + (need_ + opt_) / 4;
+        if (opt_ && hipMalloc(&h_->arena, cap) != hipSuccess) {   // no room: without the optional part
+            (void)hipGetLastError();
+            h_->arena = nullptr;
+            opt_dropped_ = true;
+            opt_ = 0;
+            cap = need_ + need_ / 4;
+        }
+        if (!h_->arena && cap) h_->arena = dev_alloc(cap, who_);
+        if (!h_->arena && cap) return err_ = ROCKET_E_NOMEM;
         h_->arena_cap = cap;
     }
-    if (need_ > 0 && !h_->arena_held) h_->arena_held = capturing_();
+    if (need_ + opt_ > 0 && !h_->arena_held) h_->arena_held = capturing_();
     return ROCKET_OK;
 }
 

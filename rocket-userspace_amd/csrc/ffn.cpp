@@ -38,11 +38,11 @@ struct F16Product {
         L.prob[0].M = M;
         ws = gemm_ws_bytes(L);
     }
-    void want_ws(Call &c) { ws = c.want_optional(ws, true); }   // the last of the reservations
+    void want_ws(Call &c) { ws = c.want_optional(ws, true); }   // after the others
     int run(Call &c, const void *A, const void *W, void *out)
     {
         L.prob[0] = Problem{L.prob[0].M, A, W, out, nullptr, nullptr, nullptr};
-        L.ws = ws ? static_cast<int32_t *>(c.scratch(ws)) : nullptr;
+        L.ws = static_cast<int32_t *>(c.optional(ws));
         L.ws_bytes = L.ws ? ws : 0;
         return c.launch(L);
     }

@@ -60,11 +60,12 @@ public:
     // Reserve arena space before in()/out(): sum of every host operand's bytes.
     void want(const void *p, size_t bytes);
     void want_scratch(size_t bytes) { need_ += round_(bytes); }
-    // Scratch that the launch can do without (K slices' planes, key splits' partials): `bytes`,
-    // reserved, or 0. While the handle's stream is being captured that is 0 where the arena would have
+    // Scratch that the launch can do without (K slices' planes, key splits' partials, a padded mask):
+    // `bytes`, reserved, or 0. While the handle's stream is being captured that is 0 where the arena would have
     // to grow, which a capture does not allow, and where the call has no other scratch, unless it is
-    // `worth` it: a graph that holds scratch of the handle must not run beside its other work. The
-    // last of the reservations.
+    // `worth` it: a graph that holds scratch of the handle must not run beside its other work. After
+    // the call's other reservations; taken with optional(), which returns null where begin() found
+    // no memory for it.
     size_t want_optional(size_t bytes, bool worth);
     // Grows the arena if needed. One that a captured call has used is kept until the handle closes:
     // the graph replays on it (each at least 1.25 times the last, so all of them at most 5 times it).
@@ -72,6 +73,7 @@ public:
     void *in(const void *p, size_t bytes);  // device view of an input
     void *out(void *p, size_t bytes);       // device view of an output
     void *scratch(size_t bytes);            // arena scratch (not copied)
+    void *optional(size_t bytes) { return bytes && !opt_dropped_ ? scratch(bytes) : nullptr; }
     int  launch(const Launch &L);           // enqueue one GEMM launch
     int  finish();                          // copy results back and wait (unless async)
     hipStream_t stream() const { return h_->stream; }
@@ -89,7 +91,8 @@ private:
     double t_stage_ = 0, t_submit_ = 0, t_wait_ = 0, t_read_ = 0;
     Handle *h_;
     const char *who_;
-    size_t need_ = 0, used_ = 0;
+    size_t need_ = 0, opt_ = 0, used_ = 0;
+    bool opt_dropped_ = false;
     bool host_io_ = false;
     int err_ = 0;
     struct Back { void *dst; const void *src; size_t bytes; };

@@ -193,7 +193,7 @@ int run(int fd, const Req &r)
         ws = c.want_optional(ws, r.fa == Fmt::F16 || r.N >= 256);
     }
     if (int rc = c.begin()) return rc;
-    int32_t *wsp = ws ? static_cast<int32_t *>(c.scratch(ws)) : nullptr;
+    int32_t *wsp = static_cast<int32_t *>(c.optional(ws));
 
     // launches hold up to kMaxProblems problems each
     for (int p0 = 0; p0 < r.nprob; p0 += kMaxProblems) {

@@ -116,11 +116,34 @@ static void blocks_on_a_small_arena()
     }
 }
 
+// Memory for what a call can do without may be short: the call then runs without it.
+static void short_of_memory()
+{
+    auto &f = fake::st();
+    const int fd = open_async();
+    f.limit = 100000;
+    CHECK(bf16(fd, 300, 15360, 96) == 0);                // no K slices' planes
+    CHECK(f.launches.size() == 1);
+    CHECK(attn(fd, 1, 4096) == 0);                       // no key splits
+    CHECK(f.launches.size() == 2);
+    CHECK(bf16(fd, 128, 8192, 512) == ROCKET_E_NOMEM);   // converted rows it needs
+    // V's rows padded, the mask read as it is
+    const int T = 512, n = 3001, np = 3008, d = 64, kvh = 2;
+    auto masked = [&] { return rocket_flash_attn_fp16(fd, T, n, d, d, 2, kvh, 0.125f, 0.f, h(X), h(W), h(W), h(X), h(Y)); };
+    f.limit = (size_t)kvh * d * np * 2 * 5 / 4 + 4096;
+    f.launches.clear();
+    CHECK(masked() == 0);
+    CHECK(fake::count("k_pad_cols") == 1 && fake::count("k_flash_attn") == 1);
+    f.limit = (size_t)-1;
+    rocket_close(fd);
+}
+
 int main()
 {
     arena_kept_for_graphs();
     small_calls_hold_no_scratch();
     blocks_on_a_small_arena();
+    short_of_memory();
     if (g_fail) {
         fprintf(stderr, "arena_check: %d check(s) failed\n", g_fail);
         return 1;
