@@ -69,9 +69,10 @@ int rocket_matmul_int4_prepacked_gw_dump(rocket_i4_ctx *ctx, int M, int K, int N
 /* The same dump for the per-row-scale entries below (validation of the entry each extends,
  * then the dump arguments) and for the grouped launches: one window per product, rows
  * [row0[e], row0[e] + nrows[e]) of product e into P[e] (nrows[e] == 0: none for that
- * product). The partials come from the kernel the plain entry runs: the dump is a run-time
- * switch of the same instantiation, so the tile, group cadence and fold are the ones a call
- * without the dump uses. Group sizes above 65536 are refused (their partials are split). */
+ * product). The partials come from the kernel the plain entry runs, by the same rule on sizes:
+ * the dump is a run-time switch of the tiled kernels' instantiation, and of the few-row kernels a
+ * copy of the same source with the stores, so the tile, group cadence and fold are the ones a
+ * call without the dump uses. Group sizes above 65536 are refused (their partials are split). */
 int rocket_matmul_int8_prepacked_gw_rowscale_dump(rocket_i8_ctx *ctx, int M, int K, int N, const int8_t *A,
                                                   const float *a_row_scale, const float *b_scale, float *Cf,
                                                   rocket_i8_weights *w, int row0, int nrows, int32_t *P);

@@ -1881,6 +1881,22 @@ hipError_t dispatch_bf16(int bm, int bn, const Launch &L, const KArgs &ka, int b
 // HBM bytes of one operand row of K elements.
 long row_bytes(Fmt f, int K);
 
+// A dump window of a few-row launch's problem (Problem::dump and its rows, null: none), and the store of
+// group g's partials for column n: d[e] is row m + e, times 16 with packed int4 weights.
+struct FewDump {
+    int32_t *p;
+    int row0, rows;
+};
+template <bool I4> __device__ __forceinline__ void few_dump(const FewDump &w, int nG, int N, int g, int n, int m, i32x4 d)
+{
+    if (g >= nG) return;   // a last chunk's tail
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int r = m + e - w.row0;
+        if (r >= 0 && r < w.rows) w.p[((size_t)r * nG + g) * N + n] = I4 ? d[e] >> 4 : d[e];
+    }
+}
+
 // A plain fp16 product whose rows keep the bits of one chain over K.
 inline bool one_chain(const Launch &L) { return L.fmt_a == Fmt::F16 && (L.epi == Epi::F16 || L.epi == Epi::F32) && !L.free_sums; }
 

@@ -46,6 +46,7 @@ struct GArgs {
     const void *A[kMaxProblems], *A2[kMaxProblems], *B[kMaxProblems];
     const float *as[kMaxProblems], *bs[kMaxProblems];
     void *C[kMaxProblems];
+    FewDump dump[kMaxProblems];
 };
 
 // Waits until at most n vector-memory instructions of this wave are outstanding; n a multiple of
@@ -69,8 +70,9 @@ __device__ __forceinline__ long lo64(i32x4 v) { return (long)(((unsigned long)(u
 // PK: K of an MFMA piece (32, 64 or, int4, 128), a divisor of the group; PPG: pieces a group (1 or
 // 2: whole groups a slot, so that a slot's body has no branch and its LDS reads, MFMAs and folds
 // overlap; 0: any number, counted). RS: a scale a row. QIN: 0 int8 codes in global memory, 1 / 2 fp32 / fp16 rows that each
-// workgroup quantises by k_quant_rows' formula (act(A) * A2 where A2 is given).
-template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT>
+// workgroup quantises by k_quant_rows' formula (act(A) * A2 where A2 is given). DUMP: the partials of
+// the launch's dump windows are stored too (an instantiation of its own: the stores cost registers).
+template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT, bool DUMP>
 __global__ __launch_bounds__(512, 2) void k_stream_gw(const GArgs a)
 {
     constexpr bool I4 = FB == Fmt::I4P;
@@ -268,6 +270,7 @@ __global__ __launch_bounds__(512, 2) void k_stream_gw(const GArgs a)
     const char *const la = codes + am * kp;
     int slot = 0;
     const int npc = K / PK;    // pieces in all
+    [[maybe_unused]] const FewDump dw = a.dump[p];
     for (int sl = sl0; sl < sl1; sl++) {
         wait_vm_le(min(max(PRE, min(depth, own)) - 1, max(PRE, own) - 1 - (sl - sl0)) * kCH);
         asm volatile("" ::: "memory");   // no read of the slot above the wait
@@ -312,6 +315,9 @@ __global__ __launch_bounds__(512, 2) void k_stream_gw(const GArgs a)
                 if (PPG ? (y + 1) % (PPG ? PPG : 1) == 0 : --left == 0) {
                     const int gi = PPG ? (sl * kCH * NP + y) / (PPG ? PPG : 1) : g;
                     const float s = SPLIT ? 0.f : S[gi * 16 + r16];
+                    if constexpr (DUMP) {
+                        if (live && dw.p) few_dump<I4>(dw, nG, N, gi, n0 + r16, 4 * q, d);
+                    }
                     if constexpr (SPLIT) {
                         if (q < a.mb) *reinterpret_cast<i32x4 *>(P + ((gi * a.mb + q) * 16 + r16) * 4) = d;
                     } else if constexpr (RS) {
@@ -376,7 +382,7 @@ __global__ __launch_bounds__(512, 2) void k_stream_gw(const GArgs a)
 
 struct GPlan {
     int w, pk, np;
-    bool split = false;
+    bool split = false, dump = false;
     size_t lds;
 };
 
@@ -386,12 +392,13 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
     const bool i4 = L.fmt_b == Fmt::I4P;
     const int sk = i4 ? 128 : 64;
     if (L.epi != Epi::GW || maxM > 16 || maxM < 1 || L.kt != L.group || L.fmt_a != Fmt::I8) return false;
-    if (L.qa && (!L.rowscale || (L.qa == 2 && i4))) return false;
+    if (L.qa && (!L.rowscale || (L.qa == 2 && i4) || L.prob[0].dump)) return false;   // (no entry dumps rows it quantises)
     if (64 * row_bytes(L.fmt_a, L.K) >= (1L << 31)) return false;   // (refused by the tiled kernels' own check)
-    for (int i = 0; i < L.nprob; i++)
-        if (L.prob[i].dump) return false;
     g.np = 0;
-    for (int i = 0; i < L.nprob; i++) g.np += L.prob[i].M > 0;
+    for (int i = 0; i < L.nprob; i++) {
+        g.np += L.prob[i].M > 0;
+        g.dump |= L.prob[i].dump != nullptr;
+    }
     g.pk = L.group % sk == 0 ? sk : (L.group % 64 == 0 ? 64 : 32);
     a.ppg = L.group / g.pk;
     a.mb = (maxM + 3) / 4;
@@ -441,9 +448,9 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
     return !L.qa || (long)maxM * L.K <= 120L * g.w * 64;
 }
 
-template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT> hipError_t launch_s(const GArgs &a, const GPlan &g, hipStream_t s)
+template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT, bool DUMP> hipError_t launch_s(const GArgs &a, const GPlan &g, hipStream_t s)
 {
-    auto kern = k_stream_gw<FB, PK, PPG, RS, QIN, SPLIT>;
+    auto kern = k_stream_gw<FB, PK, PPG, RS, QIN, SPLIT, DUMP>;
     // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any thread
     // may launch, so the mask is atomic)
     static std::atomic<uint64_t> opted{0};
@@ -462,9 +469,15 @@ template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT> hipError_t laun
 
 template <Fmt FB, int PK, int PPG, bool RS, int QIN> hipError_t launch_k(const GArgs &a, const GPlan &g, hipStream_t s)
 {
+    if constexpr (QIN == 0)
+        if (g.dump) {
+            if constexpr (PPG != 0)
+                if (g.split) return launch_s<FB, PK, PPG, RS, QIN, true, true>(a, g, s);
+            return launch_s<FB, PK, PPG, RS, QIN, false, true>(a, g, s);
+        }
     if constexpr (PPG != 0)
-        if (g.split) return launch_s<FB, PK, PPG, RS, QIN, true>(a, g, s);
-    return launch_s<FB, PK, PPG, RS, QIN, false>(a, g, s);
+        if (g.split) return launch_s<FB, PK, PPG, RS, QIN, true, false>(a, g, s);
+    return launch_s<FB, PK, PPG, RS, QIN, false, false>(a, g, s);
 }
 
 template <Fmt FB, int PK, int PPG> hipError_t launch_q(const GArgs &a, const GPlan &g, bool rs, int qa, hipStream_t s)
@@ -514,6 +527,7 @@ hipError_t stream_gw_launch(const Launch &L, int maxM, uint64_t *blocks)
         a.as[n] = P.a_scale;
         a.bs[n] = P.b_scale;
         a.C[n] = P.C;
+        a.dump[n] = FewDump{P.dump, P.dump_row0, P.dump_rows};
         n++;
     }
     *blocks = (uint64_t)(g.split ? a.nbn : (a.nbn + g.w - 1) / g.w) * g.np;

@@ -31,13 +31,15 @@ struct MArgs {
     const void *A[kMaxProblems], *B[kMaxProblems];
     const float *as[kMaxProblems], *bs[kMaxProblems];
     void *C[kMaxProblems];
+    FewDump dump[kMaxProblems];
 };
 
 __device__ __forceinline__ long pair64(int a, int b) { return (long)(((unsigned long)(unsigned)b << 32) | (unsigned)a); }
 
 // PK: K of an MFMA piece (32, 64 or, int4, 128); a group is PPG pieces (1, or 2 of a whole step: whole
-// groups a chunk). RS: a scale a row. MB: 16-row blocks a workgroup. Two or four waves.
-template <Fmt FB, int PK, int PPG, bool RS, int MB>
+// groups a chunk). RS: a scale a row. MB: 16-row blocks a workgroup. Two or four waves. DUMP: the
+// partials of the launch's dump windows are stored too.
+template <Fmt FB, int PK, int PPG, bool RS, int MB, bool DUMP>
 __global__ __launch_bounds__(256, 2) void k_mid_gw(const MArgs a)
 {
     constexpr bool I4 = FB == Fmt::I4P;
@@ -143,6 +145,7 @@ __global__ __launch_bounds__(256, 2) void k_mid_gw(const MArgs a)
     i32x4 d[MB];
 #pragma unroll
     for (int i = 0; i < MB; i++) acc[i] = f32x4{};
+    [[maybe_unused]] const FewDump dw = a.dump[p];
     for (int ch = 0; ch < nch; ch++) {
         // chunk ch has arrived (only the next chunk's instructions are outstanding; none once nothing more
         // was issued), in every wave after the barrier; every wave has read chunk ch - 1, whose place
@@ -208,6 +211,9 @@ __global__ __launch_bounds__(256, 2) void k_mid_gw(const MArgs a)
                     const float s = S[g * 16 + r16];
 #pragma unroll
                     for (int i = 0; i < MB; i++) {
+                        if constexpr (DUMP) {
+                            if (live && dw.p) few_dump<I4>(dw, nG, N, g, n0 + r16, m0 + 16 * i + 4 * q, d[i]);
+                        }
                         if constexpr (RS) {
 #pragma unroll
                             for (int e = 0; e < 4; e++) acc[i][e] = __builtin_fmaf(s, (float)d[i][e], acc[i][e]);
@@ -238,6 +244,7 @@ __global__ __launch_bounds__(256, 2) void k_mid_gw(const MArgs a)
 
 struct MPlan {
     int w, pk, np, mb, nb;
+    bool dump = false;
     size_t lds;
 };
 
@@ -251,8 +258,8 @@ bool plan_mid(const Launch &L, int maxM, MPlan &g, MArgs &a)
     if ((long)maxM * a.nbn > 256L * 32 * 8) return false;   // past every form below, whatever the rest says
     g.np = 0;
     for (int i = 0; i < L.nprob; i++) {
-        if (L.prob[i].dump) return false;
         g.np += L.prob[i].M > 0;
+        g.dump |= L.prob[i].dump != nullptr;
     }
     g.pk = L.group % sk == 0 ? sk : (L.group % 64 == 0 ? 64 : 32);
     a.ppg = L.group / g.pk;
@@ -283,9 +290,9 @@ bool plan_mid(const Launch &L, int maxM, MPlan &g, MArgs &a)
     return false;
 }
 
-template <Fmt FB, int PK, int PPG, bool RS, int MB> hipError_t launch_mid_k(const MArgs &a, const MPlan &g, hipStream_t s)
+template <Fmt FB, int PK, int PPG, bool RS, int MB, bool DUMP> hipError_t launch_mid_k(const MArgs &a, const MPlan &g, hipStream_t s)
 {
-    auto kern = k_mid_gw<FB, PK, PPG, RS, MB>;
+    auto kern = k_mid_gw<FB, PK, PPG, RS, MB, DUMP>;
     // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any thread
     // may launch, so the mask is atomic)
     static std::atomic<uint64_t> opted{0};
@@ -307,7 +314,9 @@ template <Fmt FB, int PK> hipError_t launch_mid_pk(const MArgs &a, const MPlan &
     auto by = [&](auto PPG, auto RS) {
         constexpr int P = decltype(PPG)::value;
         constexpr bool R = decltype(RS)::value;
-        return g.mb == 1 ? launch_mid_k<FB, PK, P, R, 1>(a, g, L.stream) : launch_mid_k<FB, PK, P, R, 2>(a, g, L.stream);
+        if (g.dump)
+            return g.mb == 1 ? launch_mid_k<FB, PK, P, R, 1, true>(a, g, L.stream) : launch_mid_k<FB, PK, P, R, 2, true>(a, g, L.stream);
+        return g.mb == 1 ? launch_mid_k<FB, PK, P, R, 1, false>(a, g, L.stream) : launch_mid_k<FB, PK, P, R, 2, false>(a, g, L.stream);
     };
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
@@ -344,6 +353,7 @@ hipError_t mid_gw_launch(const Launch &L, int maxM, uint64_t *blocks)
         a.as[n] = P.a_scale;
         a.bs[n] = P.b_scale;
         a.C[n] = P.C;
+        a.dump[n] = FewDump{P.dump, P.dump_row0, P.dump_rows};
         n++;
     }
     *blocks = (uint64_t)((a.nbn + g.w - 1) / g.w) * g.np * g.nb;

@@ -1,5 +1,5 @@
-// arena_check.cpp — what the library's calls do with a handle's scratch, on the fake runtime of
-// fake_hip.h: which kernels a call launches where the arena may not grow (a captured stream), what a
+// arena_check.cpp — what the library's calls launch and do with a handle's scratch, on the fake runtime
+// of fake_hip.h: which kernels a call launches where the arena may not grow (a captured stream), what a
 // captured call's graph may still replay on after the arena has grown, and what is freed when the
 // handle closes. Built and run by tests/test_arena.py. Exit status 0 when every check passes.
 #include "fake_hip.h"
@@ -138,12 +138,38 @@ static void short_of_memory()
     rocket_close(fd);
 }
 
+// A dump's partials come from the kernel that the call without it runs.
+static void dumps_run_the_same_kernel()
+{
+    auto &f = fake::st();
+    const int fd = open_async();
+    int8_t *const A = reinterpret_cast<int8_t *>(X), *const B = reinterpret_cast<int8_t *>(W);
+    for (int M : {4, 16, 20, 64, 512})
+        for (int N : {64, 4096}) {
+            auto base = [&] {
+                // the name up to its template arguments (the last of which is the dump)
+                CHECK(f.launches.size() == 1);
+                std::string n = f.launches.empty() ? "" : f.launches[0];
+                const size_t at = n.find("k_");
+                return at == std::string::npos ? n : n.substr(at, n.find('I', at) - at);
+            };
+            f.launches.clear();
+            CHECK(rocket_matmul_int8_groupwise(fd, M, 1024, N, A, B, X, W, Y, 128) == 0);
+            const std::string plain = base();
+            f.launches.clear();
+            CHECK(rocket_matmul_int8_groupwise_dump(fd, M, 1024, N, A, B, X, W, Y, 128, 0, 4, reinterpret_cast<int32_t *>(Y)) == 0);
+            CHECK(base() == plain && !plain.empty());
+        }
+    rocket_close(fd);
+}
+
 int main()
 {
     arena_kept_for_graphs();
     small_calls_hold_no_scratch();
     blocks_on_a_small_arena();
     short_of_memory();
+    dumps_run_the_same_kernel();
     if (g_fail) {
         fprintf(stderr, "arena_check: %d check(s) failed\n", g_fail);
         return 1;

@@ -14,6 +14,14 @@ import rocketnpu as R
 pytestmark = pytest.mark.gpu
 SEED = 0x52434B80
 
+
+
+def partials(A, B, group):
+    """P[m][g][n]: the sums of every group, below 2^24 for groups of up to 1023 and exact in fp32."""
+    a, b = A.astype(np.float32), B.astype(np.float32)
+    return np.stack([a[:, k:k + group] @ b[:, k:k + group].T for k in range(0, A.shape[1], group)], 1).astype(np.int32)
+
+
 SHAPES = [(4, 64, 64, 32), (4, 128, 64, 128), (8, 608, 128, 32), (16, 576, 192, 64), (20, 608, 128, 32), (12, 768, 128, 96),
           (4, 2048, 128, 256), (16, 2048, 64, 512), (16, 4096, 64, 32), (4, 8448, 64, 128), (8, 256, 8256, 32),
           (12, 1152, 8320, 128), (16, 512, 8256, 64), (4, 640, 8256, 160)]
@@ -38,9 +46,19 @@ def test_stream_gw(lib, orc, M, K, N, group, int4):
     out = np.full((M, N), np.nan, np.float32)
     assert call("_rowscale", R.ptr(A), R.ptr(row), R.ptr(bsc), R.ptr(out)) == 0
     assert np.array_equal(out, orc.matmul_gw_rowscale_f32(A, B, row, bsc, group))
+    plain = out.copy()
     out[:] = np.nan
     assert call("", R.ptr(A), R.ptr(asc), R.ptr(bsc), R.ptr(out)) == 0
     assert np.array_equal(out, gworder.gw_f32(orc, A, B, asc, bsc, group))
+    # the same kernels with their partials dumped: a window of rows inside the blocks
+    r0, nr = (13, 6) if M > 16 else (1, M - 2)
+    want = partials(A[r0:r0 + nr], B, group)
+    for name, scale, first in (("_rowscale_dump", row, plain), ("_dump", asc, out.copy())):
+        P = np.full((nr, nG, N), 99, np.int32)
+        out[:] = np.nan
+        assert getattr(lib, f"rocket_matmul_int{4 if int4 else 8}_prepacked_gw{name}")(
+            ctx, M, K, N, R.ptr(A), R.ptr(scale), R.ptr(bsc), R.ptr(out), w, r0, nr, R.ptr(P)) == 0
+        assert np.array_equal(out, first) and np.array_equal(P, want)
     x = orc.gen_normal((M, K), SEED + 6)
     x[2] = 0.0                  # a row of zeros: codes and scale 0
     q, s = orc.quant_rows(x)
@@ -86,6 +104,35 @@ def test_stream_gw_grouped(lib, orc, Ms, K, N, group):
             x = (orc.f16_bits_to_f32(G[e][:m]) * orc.f16_bits_to_f32(U[e][:m])).astype(np.float32)
             q, s = orc.quant_rows(x)
             assert np.array_equal(out[e][:m], orc.matmul_gw_rowscale_f32(q, Bs[e], s, bs[e], group))
+    del k0, k1, k2, k3, k4, k5, k6, k7
+    for w in W:
+        lib.rocket_i8_weights_free(ctx, w)
+    lib.rocket_i8_ctx_free(ctx)
+
+
+@pytest.mark.parametrize("Ms,group", [([4, 0, 16, 8], 32), ([4, 20, 32], 64)])
+def test_few_rows_grouped_dump(lib, orc, Ms, group):
+    """Windows of some products of a grouped launch and none of the others, few rows and more."""
+    K, N, n = 512, 96, len(Ms)
+    print(f"few rows grouped dump Ms={Ms} group={group}", flush=True)
+    nG = K // group
+    ctx = lib.rocket_i8_ctx_create(1)
+    Bs, A = [orc.gen_i8((N, K), SEED + 200 + e) for e in range(n)], [orc.gen_i8((max(m, 4), K), SEED + 220 + e) for e, m in enumerate(Ms)]
+    W = [lib.rocket_i8_weights_pack_gw(ctx, 4, K, N, R.ptr(b), group) for b in Bs]
+    bs = [orc.gen_uniform((N, nG), SEED + 240 + e, 0.005, 0.02) for e in range(n)]
+    rs = [orc.gen_uniform((max(m, 4),), SEED + 260 + e, 0.5, 1.5) for e, m in enumerate(Ms)]
+    out, P = [np.full((max(m, 4), N), np.nan, np.float32) for m in Ms], [np.full((3, nG, N), 99, np.int32) for _ in Ms]
+    r0, nr = [1] * n, [3 if e != 0 and m else 0 for e, m in enumerate(Ms)]
+    pW = C.cast((C.c_void_p * n)(*W), R.pp)
+    (pM, k0), (pr0, k1), (pnr, k2) = R.int_array(Ms), R.int_array(r0), R.int_array(nr)
+    (pA, k3), (pr, k4), (pb, k5), (po, k6), (pP, k7) = (R.ptr_array(x) for x in (A, rs, bs, out, P))
+    assert lib.rocket_matmul_int8_prepacked_gw_grouped_rowscale_dump(ctx, n, pM, K, N, pA, pr, pb, po, pW, pr0, pnr, pP) == 0
+    for e, m in enumerate(Ms):
+        if m:
+            assert np.array_equal(out[e][:m], orc.matmul_gw_rowscale_f32(np.ascontiguousarray(A[e][:m]), Bs[e],
+                                                                         np.ascontiguousarray(rs[e][:m]), bs[e], group))
+        want = partials(A[e], Bs[e], group)[1:4] if nr[e] else 99
+        assert np.all(P[e] == want)
     del k0, k1, k2, k3, k4, k5, k6, k7
     for w in W:
         lib.rocket_i8_weights_free(ctx, w)

@@ -12,6 +12,7 @@ import pytest
 
 import gworder
 import rocketnpu as R
+from test_gpu_stream_gw import partials
 
 pytestmark = pytest.mark.gpu
 SEED = 0x52434D80
@@ -42,9 +43,19 @@ def test_stream_gw_mid(lib, orc, M, K, N, group, int4):
     out = np.full((M, N), np.nan, np.float32)
     assert call("_rowscale", R.ptr(A), R.ptr(row), R.ptr(bsc), R.ptr(out)) == 0
     assert np.array_equal(out, orc.matmul_gw_rowscale_f32(A, B, row, bsc, group))
+    plain = out.copy()
     out[:] = np.nan
     assert call("", R.ptr(A), R.ptr(asc), R.ptr(bsc), R.ptr(out)) == 0
     assert np.array_equal(out, gworder.gw_f32(orc, A, B, asc, bsc, group))
+    # the same kernels with their partials dumped: a window of rows inside the blocks
+    r0, nr = (13, 6) if M > 16 else (1, M - 2)
+    want = partials(A[r0:r0 + nr], B, group)
+    for name, scale, first in (("_rowscale_dump", row, plain), ("_dump", asc, out.copy())):
+        P = np.full((nr, nG, N), 99, np.int32)
+        out[:] = np.nan
+        assert getattr(lib, f"rocket_matmul_int{4 if int4 else 8}_prepacked_gw{name}")(
+            ctx, M, K, N, R.ptr(A), R.ptr(scale), R.ptr(bsc), R.ptr(out), w, r0, nr, R.ptr(P)) == 0
+        assert np.array_equal(out, first) and np.array_equal(P, want)
     getattr(lib, f"rocket_{kind}_weights_free")(ctx, w)
     getattr(lib, f"rocket_{kind}_ctx_free")(ctx)
 
