@@ -356,8 +356,9 @@ __global__ __launch_bounds__(512, 2) void k_stream_gw(const GArgs a)
             for (int e = 0; e < 8; e++) {
                 const int gg = min(g8 + e, nGp - 1);
                 pv[e] = P[gg * (a.mb * 64) + tid];
-                s[e] = g8 + e < nGp ? S[gg * 16 + fn] : 0.f;
+                s[e] = S[gg * 16 + fn];
                 if constexpr (!RS) s[e] *= AS[gg * 16 + fm];
+                if (g8 + e >= nGp) s[e] = 0.f;   // (the product: a last group's scale may be infinite)
             }
 #pragma unroll
             for (int e = 0; e < 8; e++) f = __builtin_fmaf(s[e], (float)pv[e], f);

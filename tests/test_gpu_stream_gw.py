@@ -137,3 +137,26 @@ def test_few_rows_grouped_dump(lib, orc, Ms, group):
     for w in W:
         lib.rocket_i8_weights_free(ctx, w)
     lib.rocket_i8_ctx_free(ctx)
+
+
+@pytest.mark.parametrize("M,K,N,group", [(4, 1536, 64, 128), (8, 2560, 192, 128), (4, 1536, 8256, 128), (20, 1536, 64, 128), (12, 640, 64, 64)])
+@pytest.mark.parametrize("int4", [True, False])
+def test_infinite_activation_scales(lib, orc, M, K, N, group, int4):
+    """An infinite scale of one group (the last, where the groups are no multiple of eight; the first; one
+    row's only scale) gives the chain's infinities, and no NaN where the chain has none."""
+    print(f"infinite scales int4={int4} M={M} K={K} N={N} group={group}", flush=True)
+    nG, kind = K // group, "i4" if int4 else "i8"
+    A, B = orc.gen_i8((M, K), SEED + 300, 1, 127), orc.gen_i8((N, K), SEED + 301, 1, 7)     # partials above 0
+    bsc = orc.gen_uniform((N, nG), SEED + 302, 0.005, 0.02)
+    asc = orc.gen_uniform((M, nG), SEED + 303, 0.5, 1.5)
+    asc[0, -1], asc[1, 0], asc[2, :] = np.inf, np.inf, np.inf
+    want = gworder.gw_f32(orc, A, B, asc, bsc, group)
+    assert np.isinf(want[:3]).all() and np.isfinite(want[3:]).all()
+    ctx = getattr(lib, f"rocket_{kind}_ctx_create")(1)
+    w = getattr(lib, f"rocket_{kind}_weights_pack_gw")(ctx, 4, K, N, R.ptr(B), group)
+    out = np.full((M, N), np.nan, np.float32)
+    fn = getattr(lib, f"rocket_matmul_int{4 if int4 else 8}_prepacked_gw")
+    assert fn(ctx, M, K, N, R.ptr(A), R.ptr(asc), R.ptr(bsc), R.ptr(out), w) == 0
+    assert np.array_equal(out, want)
+    getattr(lib, f"rocket_{kind}_weights_free")(ctx, w)
+    getattr(lib, f"rocket_{kind}_ctx_free")(ctx)
