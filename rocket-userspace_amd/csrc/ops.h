@@ -42,6 +42,9 @@ struct Req {
 // Runs a request on handle fd: stages host operands, launches, copies back, waits.
 int run(int fd, const Req &r);
 
+// Whether a result of the request lies over rows (A, A2) of it: a_row bytes a row, c_elem a result.
+bool results_overlap_rows(const Req &r, size_t a_row, size_t c_elem);
+
 // Bytes of one operand row in HBM for a format.
 size_t fmt_row_bytes(Fmt f, int K);
 // Bytes of one C element for an epilogue.

@@ -6,6 +6,11 @@
 
 #include <stdio.h>
 
+#include <algorithm>
+#include <chrono>
+#include <random>
+
+#include "ops.h"
 #include "rocket_attn.h"
 #include "rocket_ffn.h"
 #include "rocket_hip.h"
@@ -163,6 +168,60 @@ static void dumps_run_the_same_kernel()
     rocket_close(fd);
 }
 
+// Results over rows, against every pair; and in a time that grows with the products, not their square.
+static void overlaps()
+{
+    std::mt19937 rng(7);
+    std::vector<int> M;
+    std::vector<const void *> A, A2;
+    std::vector<void *> C;
+    rk::Req r;
+    auto make = [&](int n, int spread) {
+        M.resize(n), A.resize(n), A2.resize(n), C.resize(n);
+        for (int i = 0; i < n; i++) {
+            M[i] = (int)(rng() % 4) * 4;
+            A[i] = (const void *)(uintptr_t)(4096 + rng() % spread * 16);
+            A2[i] = (const void *)(uintptr_t)(4096 + rng() % spread * 16);
+            C[i] = (void *)(uintptr_t)(4096 + rng() % spread * 16);
+        }
+        r.nprob = n;
+        r.N = 32;
+        r.M = M.data(), r.A = A.data(), r.C = C.data();
+        r.A2 = rng() % 2 ? A2.data() : nullptr;
+    };
+    int hits = 0;
+    for (int t = 0; t < 4000; t++) {
+        make(1 + (int)(rng() % 20), 40 << (rng() % 10));
+        bool any = false;
+        const size_t row = 64, el = 4;
+        for (int p = 0; p < r.nprob; p++)
+            for (int q = 0; q < r.nprob; q++)
+                for (const void *a : {A[p], r.A2 ? A2[p] : A[p]}) {
+                    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)C[q];
+                    if (M[p] && M[q] && x < y + (size_t)M[q] * r.N * el && y < x + M[p] * row) any = true;
+                }
+        CHECK(rk::results_overlap_rows(r, row, el) == any);
+        hits += any;
+    }
+    CHECK(hits > 400 && hits < 3600);
+    auto time = [&](int n) {   // rows and results in turn in memory, none over another
+        make(n, 1);
+        for (int i = 0; i < n; i++) {
+            M[i] = 4;
+            A[i] = A2[i] = (const void *)(uintptr_t)(4096 + 4096 * (size_t)(2 * i));
+            C[i] = (void *)(uintptr_t)(4096 + 4096 * (size_t)(2 * i + 1));
+        }
+        double best = 1e9;
+        for (int k = 0; k < 9; k++) {
+            const auto t0 = std::chrono::steady_clock::now();
+            CHECK(!rk::results_overlap_rows(r, 64, 4));
+            best = std::min(best, std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+        }
+        return best;
+    };
+    CHECK(time(4096) < 100 * time(128));   // 32 times the products: their square takes 1024 times as long
+}
+
 int main()
 {
     arena_kept_for_graphs();
@@ -170,6 +229,7 @@ int main()
     blocks_on_a_small_arena();
     short_of_memory();
     dumps_run_the_same_kernel();
+    overlaps();
     if (g_fail) {
         fprintf(stderr, "arena_check: %d check(s) failed\n", g_fail);
         return 1;

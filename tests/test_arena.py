@@ -17,7 +17,8 @@ def test_scratch_under_growth_and_capture(tmp_path):
     if not os.path.exists(cxx) or not os.path.exists(lib) or not os.path.exists(src):
         pytest.skip("needs clang++ and the static library")
     exe = str(tmp_path / "arena_check")
-    b = subprocess.run([cxx, "-std=c++17", "-O1", "-I", os.path.join(REPO, "include"), "-I/opt/rocm/include", src, lib, "-o", exe,
+    b = subprocess.run([cxx, "-std=c++17", "-O1", "-I", os.path.join(REPO, "include"), "-I", os.path.join(PKG, "csrc"),
+                        "-I/opt/rocm/include", src, lib, "-o", exe,
                         "-lm", "-lpthread"], capture_output=True, text=True, timeout=300)
     assert b.returncode == 0, b.stdout[-3000:] + b.stderr[-3000:]
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
