@@ -429,7 +429,7 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
         // as two (16 rows, 3840 x 15360: 11.9 us with four waves, 22.1 with two, which leave one
         // workgroup a CU; the MoE's 1408 gate and up tiles: 29.1 with two, 35.1 with four).
         a.depth = 3;
-        int best = 0;
+        int best = 0, waves = 0, rounds = 0;   // of the best: waves a CU, batches of workgroups
         for (int w = 8; w >= 1; w /= 2) {
             const size_t b = shared + w * (tab + a.depth * slot);
             if (b > lds) continue;
@@ -439,9 +439,18 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
                 best = cost;
                 g.w = w;
                 g.lds = b;
+                waves = w * fit;
+                rounds = (each + fit - 1) / fit;
             }
         }
         if (!best) return false;
+        // Long rows leave LDS for one or two waves a CU, and several batches of those take longer than
+        // the tiles: int4, from more batches than waves (16 x 8192 x 16384, groups of 128, one wave, four
+        // batches: 90.6 us, tiles 44.2; 16 x 8192 x 12288, groups of 256, two and two: 38.1 and 33.4; 16 x
+        // 5120 x 16384, groups of 32, two and two: 39.7 and 49.5); int8, whose tiles unpack nothing, from
+        // two (16 x 8192 x 16384, groups of 32: 153.7, tiles 43.4; 16 x 8192 x 16384, groups of 256, two
+        // waves and two batches: 57.6 and 42.9; four waves and two batches at the least 1.06 of the tiles').
+        if (i4 ? rounds > waves : rounds > 1 && waves <= 2) return false;
     }
     // Rows are quantised here while a thread has at most 120 elements of them; more of it in every
     // workgroup costs what the pass ahead does (fp32 rows, 3840 x 15360: 4 rows 15.6 -> 13.4 us, 8

@@ -222,6 +222,35 @@ static void overlaps()
     CHECK(time(4096) < 100 * time(128));   // 32 times the products: their square takes 1024 times as long
 }
 
+// The kernels that sizes on both sides of a dispatch rule's line run.
+static void routes()
+{
+    const int fd = open_async();
+    int8_t *const A = reinterpret_cast<int8_t *>(X), *const B = reinterpret_cast<int8_t *>(W);
+    auto ran = [&](const char *kernel) {
+        const bool r = fake::count(kernel) == 1;
+        if (!r)
+            for (const auto &l : fake::st().launches) fprintf(stderr, "  launched %s\n", l.c_str());
+        fake::st().launches.clear();
+        return r;
+    };
+    auto gw8 = [&](int M, int K, int N, int g) { return rocket_matmul_int8_groupwise(fd, M, K, N, A, B, X, W, Y, g) == 0; };
+    auto gw4 = [&](int M, int K, int N, int g) { return rocket_matmul_int4_groupwise(fd, M, K, N, A, B, X, W, Y, g) == 0; };
+    auto int8 = [&](int M, int K, int N) { return rocket_matmul_int8(fd, M, K, N, A, B, reinterpret_cast<int32_t *>(Y)) == 0; };
+    auto tf32 = [&](int M, int K, int N) { return rocket_matmul_tf32(fd, M, K, N, X, W, Y) == 0; };
+    auto fa = [&](int T, int n, int d, int heads, int kv) {
+        return rocket_flash_attn_fp16(fd, T, n, d, d, heads, kv, 0.1f, 0.f, h(X), h(W), h(W), nullptr, h(Y)) == 0;
+    };
+    (void)gw8, (void)gw4, (void)int8, (void)tf32, (void)fa;
+    // rows so long that LDS holds a wave or two a CU
+    CHECK(gw4(16, 8192, 4096, 128) && ran("k_stream_gw"));
+    CHECK(gw4(16, 8192, 16384, 128) && ran("k_gemm"));
+    CHECK(gw8(16, 4096, 16384, 32) && ran("k_stream_gw"));
+    CHECK(gw8(16, 8192, 16384, 32) && ran("k_gemm"));
+    CHECK(gw8(16, 8192, 8192, 64) && ran("k_gemm"));
+    rocket_close(fd);
+}
+
 int main()
 {
     arena_kept_for_graphs();
@@ -230,6 +259,7 @@ int main()
     short_of_memory();
     dumps_run_the_same_kernel();
     overlaps();
+    routes();
     if (g_fail) {
         fprintf(stderr, "arena_check: %d check(s) failed\n", g_fail);
         return 1;
