@@ -271,10 +271,16 @@ bool plan_mid(const Launch &L, int maxM, MPlan &g, MArgs &a)
     // holds at once are the tiles' (256 x 3840 x 15360: 50, tiles 35.9). 64 rows a workgroup were
     // slower than the tiles with groups of 32 (396 x 4608 x 1344: 43.3, tiles 39.9), and so are two a CU
     // of int8 weights with such groups, four folds a step (MoE layers of 132 and 194 tokens, hidden 2880
-    // and 2944: 41.6 and 43.1, tiles 38.8 and 39.0).
+    // and 2944: 41.6 and 43.1, tiles 38.8 and 39.0). Of int8 weights two a CU, and with groups of 32 one a
+    // CU of many columns, keep ahead of the tiles on short rows alone (64 x 16384, groups of 64: K = 1024
+    // 1.06 times as fast, 2048 0.98, 4096 0.89, 8192 51.0 us against 42.9; 128 x 8192, groups of 128: 1.10,
+    // 0.99, 0.91, 0.86; 64 x 8192, groups of 32: 1.12, 0.98, 0.91, 0.85; at 6144 columns 1.29 to 1.17), or
+    // where a tile's 64 rows are half empty (MoE layers of 64 tokens, hidden 4096, groups of 64: 56.2, tiles
+    // 73.9).
     static const int form[][2] = {{1, 1}, {2, 1}, {2, 2}};
     for (const auto &f : form) {
         if (f[1] == 2 && !i4 && L.group < 64) continue;
+        if (!i4 && L.K > 2048 && ((f[1] == 2 && maxM > 32) || (f[0] == 2 && L.group < 64 && L.N >= 8192))) continue;
         g.mb = f[0];
         const int chunk = sk * mid_steps(g.mb);
         a.nch = (L.K + chunk - 1) / chunk;
