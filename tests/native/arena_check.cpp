@@ -253,6 +253,14 @@ static void routes()
     CHECK(gw8(64, 8192, 16384, 64) && ran("k_gemm"));
     CHECK(gw8(48, 8192, 6144, 32) && ran("k_mid_gw"));
     CHECK(gw8(48, 8192, 8192, 32) && ran("k_gemm"));
+    // int8 to int32, few rows
+    CHECK(int8(16, 8192, 4096) && ran("k_stream"));
+    CHECK(int8(16, 8192, 8192) && ran("k_gemm"));
+    CHECK(int8(4, 8192, 8192) && ran("k_stream"));
+    CHECK(int8(4, 4096, 16384) && ran("k_gemm"));
+    CHECK(int8(4, 4096, 24576) && ran("k_stream"));
+    CHECK(int8(4, 512, 16384) && ran("k_stream"));
+    CHECK(int8(4, 512, 32768) && ran("k_gemm"));
     rocket_close(fd);
 }
 
