@@ -129,8 +129,16 @@ int f32_prepass(const Req &r)
     for (int p = 0; p < r.nprob; p++) maxM = std::max(maxM, r.M[p]);
     // (with few columns, or few values, the pass's own launch costs more than it saves: tf32 700 x
     // 2528 x 272 25.6 us with it, 20.3 without; 128 x 2048 x 2048 17.5 and 16.0; 128 x 4096 x 4096
-    // 30.6 and 33.4)
-    bool pays = r.N >= 384 && (long)maxM * r.K >= 400000;
+    // 30.6 and 33.4. Few values that many columns' tiles read again are worth it all the same: tf32 256 x
+    // 1024 x 8192 25.1 with it, 27.7 without; 2044 x 128 x 8192 35.7 and 42.2; 20 x 2048 x 16384 39.1 and
+    // 48.3; 64 x 2048 x 8192 22 and 21.2; bf16, whose conversion in the loads is cheaper, 512 x 512 x
+    // 16384 24.8 and 27.7; 64 x 4096 x 8192 35.0 and 45.5; 256 x 512 x 8192 13 and 12)
+    const long mk = (long)maxM * r.K;
+    bool pays = r.N >= 384 && mk >= 400000;
+    if (r.fa == Fmt::F32TF32)
+        pays = pays || (r.N >= 8192 && ((maxM >= 128 && mk * r.N >= 1000000000L) || (r.K >= 512 && (r.K <= 1024 || r.N >= 16384))));
+    else
+        pays = pays || (r.N >= 384 && mk * r.N >= 4000000000L) || (r.N >= 4096 && r.N < 16384 && r.K >= 2048 && mk >= 80000);
     Launch L;   // few rows: the weight-streaming kernel converts as it loads
     L.fmt_a = r.fa; L.fmt_b = r.fb; L.epi = r.epi; L.N = r.N; L.K = L.kend = r.K;
     L.nprob = 1;

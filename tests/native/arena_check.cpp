@@ -261,6 +261,13 @@ static void routes()
     CHECK(int8(4, 4096, 24576) && ran("k_stream"));
     CHECK(int8(4, 512, 16384) && ran("k_stream"));
     CHECK(int8(4, 512, 32768) && ran("k_gemm"));
+    // fp32 rows converted ahead
+    CHECK(tf32(128, 2048, 2048) && !ran("k_cvt"));
+    CHECK(tf32(128, 4096, 4096) && ran("k_cvt"));
+    CHECK(tf32(256, 1024, 8192) && ran("k_cvt"));
+    CHECK(tf32(2044, 128, 8192) && ran("k_cvt"));
+    CHECK(tf32(20, 2048, 16384) && ran("k_cvt"));
+    CHECK(tf32(64, 2048, 8192) && !ran("k_cvt"));
     rocket_close(fd);
 }
 
