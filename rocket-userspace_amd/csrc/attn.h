@@ -35,6 +35,10 @@ constexpr int kAttnMaxHeadDim = 256;
 
 hipError_t flash_attn(const FaLaunch &L, hipStream_t s, uint64_t *blocks_out);
 
+// Whether the tiled kernel's workgroups (128 queries of a head, a share of the keys) fill the CUs in
+// whole rounds.
+bool flash_attn_tiles_fill(const FaLaunch &L);
+
 // Few query rows a KV head (attn_decode.hip): whether the launch takes the kernel for them (T,
 // n_kv, dk, dv, n_head and gqa decide), its workspace and its launch, on operands that
 // flash_attn has checked.

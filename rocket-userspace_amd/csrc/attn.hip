@@ -661,6 +661,12 @@ static int fa_splits(const FaLaunch &L)
     return want < 1 ? 1 : (int)want;
 }
 
+bool flash_attn_tiles_fill(const FaLaunch &L)
+{
+    const long wgs = (long)((L.T + BQ - 1) / BQ) * L.n_head * fa_splits(L);
+    return wgs >= 230 && (wgs % 256 == 0 || wgs % 256 >= 230);
+}
+
 size_t flash_attn_ws_bytes(const FaLaunch &L)
 {
     if (flash_attn_few_rows(L)) return flash_attn_rows_ws(L);

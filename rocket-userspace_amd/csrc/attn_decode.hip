@@ -320,11 +320,15 @@ template <int D> hipError_t launch_rows(const RowArgs &a, int kv_heads, hipStrea
     return cap ? launch_rows_f<D, true, false>(a, kv_heads, s) : launch_rows_f<D, false, false>(a, kv_heads, s);
 }
 
-// Workgroups a KV head: one chunk a wave while the workgroups stay near three a CU.
+// Workgroups a KV head: one chunk a wave while the workgroups stay near three a CU; one workgroup for
+// short caches, where the merge's launch costs more than the waves' further chunks (one token, 32 heads
+// of 64, 192 keys 4.3 us, split 7.0; 512 keys 6.4 and 7.1; heads of 128, 320 keys 7.5 and 8.3, 384 keys
+// 8.1 and 8.3; heads of 256, 256 keys 10.2 and 10.5, 320 keys 12.2 and 10.5).
 void split_of(const FaLaunch &L, int *nsplit, int *cps)
 {
     const int kvh = L.n_head / L.gqa, chunks = (L.n_kv + kChunk - 1) / kChunk;
-    int n = std::min({(chunks + kWaves - 1) / kWaves, std::max(1, 768 / kvh), 64});
+    const int d = std::max(L.dk, L.dv), whole = d <= 64 ? 16 : d <= 128 ? 10 : 8;
+    const int n = chunks <= whole ? 1 : std::min({(chunks + kWaves - 1) / kWaves, std::max(1, 768 / kvh), 64});
     *cps = (chunks + n - 1) / n;
     *nsplit = (chunks + *cps - 1) / *cps;
 }
@@ -333,7 +337,16 @@ void split_of(const FaLaunch &L, int *nsplit, int *cps)
 
 bool flash_attn_few_rows(const FaLaunch &L)
 {
-    return (long)L.gqa * L.T <= kRows && L.n_kv >= 8 && L.dk % 32 == 0 && L.dv % 16 == 0;
+    if ((long)L.gqa * L.T > kRows || L.n_kv < 8 || L.dk % 32 || L.dv % 16) return false;
+    // One query head a KV head and long caches: the tiled kernel reads V^T in whole 128-byte lines (64
+    // keys a tile, 32 here), and where its workgroups fill the CUs and nothing has to be padded it is the
+    // faster one while the cache is not far larger than the memory-side cache (heads of 256, 16 x 8192
+    // keys 28.9 us, here 33.0; 32 x 8192 54.8 and 62.8, 32 x 32768 212 and 200; heads of 128, 32 x 8192 28.3
+    // and 30.7; 24 heads, whose 264 workgroups are two rounds, 8192 keys 69 and 48.6).
+    const int d = std::max(L.dk, L.dv);
+    const size_t kv = (size_t)L.n_head / L.gqa * L.n_kv * (L.dk + L.dv) * sizeof(_Float16);
+    return !(L.gqa == 1 && d > 64 && L.n_kv % 8 == 0 && kv >= ((size_t)(d > 128 ? 64 : 96) << 20) && kv <= ((size_t)512 << 20) &&
+             flash_attn_tiles_fill(L));
 }
 
 size_t flash_attn_rows_ws(const FaLaunch &L)

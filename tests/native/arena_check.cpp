@@ -268,6 +268,15 @@ static void routes()
     CHECK(tf32(2044, 128, 8192) && ran("k_cvt"));
     CHECK(tf32(20, 2048, 16384) && ran("k_cvt"));
     CHECK(tf32(64, 2048, 8192) && !ran("k_cvt"));
+    // attention of few query rows: short caches, and long ones of one query head a KV head
+    CHECK(fa(1, 192, 128, 8, 8) && fake::st().launches.size() == 1 && ran("k_fa_rows"));
+    CHECK(fa(1, 512, 64, 8, 8) && fake::st().launches.size() == 1 && ran("k_fa_rows"));
+    CHECK(fa(1, 512, 128, 8, 8) && fake::st().launches.size() == 2 && ran("k_fa_rows"));
+    CHECK(fa(1, 8192, 256, 32, 32) && ran("k_flash_attn"));
+    CHECK(fa(1, 8191, 256, 32, 32) && ran("k_fa_rows"));
+    CHECK(fa(1, 8192, 256, 64, 32) && ran("k_fa_rows"));
+    CHECK(fa(1, 8192, 256, 24, 24) && ran("k_fa_rows"));
+    CHECK(fa(1, 8192, 64, 32, 32) && ran("k_fa_rows"));
     rocket_close(fd);
 }
 
