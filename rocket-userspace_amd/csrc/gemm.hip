@@ -560,7 +560,8 @@ bool small_takes(const Launch &L, int maxM)
     if (L.fmt_a != Fmt::F16 || L.fmt_b != Fmt::F16 || (L.epi != Epi::F16 && L.epi != Epi::F32) || L.nprob != 1 || L.accum ||
         L.kbeg != 0 || L.kend != L.K || L.K > 1024)
         return false;
-    return maxM <= 32 || (long)((maxM + 31) / 32) * ((L.N + 31) / 32) <= 64;
+    if (maxM <= 16 || (maxM <= 32 && (long)L.K * L.N <= 33000000)) return true;   // (32 x 1024 x 65536 35.8, tiles 31.6)
+    return (long)((maxM + 31) / 32) * ((L.N + 31) / 32) <= 64;
 }
 
 // [slice][M][N] planes of fp32 partials

@@ -277,6 +277,9 @@ static void routes()
     CHECK(fa(1, 8192, 256, 64, 32) && ran("k_fa_rows"));
     CHECK(fa(1, 8192, 256, 24, 24) && ran("k_fa_rows"));
     CHECK(fa(1, 8192, 64, 32, 32) && ran("k_fa_rows"));
+    // fp16, 17 to 32 rows of short K
+    CHECK(fp16(fd, 32, 992, 32768) == 0 && ran("k_small_f16"));
+    CHECK(fp16(fd, 32, 992, 65536) == 0 && ran("k_gemm"));
     rocket_close(fd);
 }
 
