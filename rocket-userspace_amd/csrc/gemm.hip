@@ -564,6 +564,22 @@ bool small_takes(const Launch &L, int maxM)
     return (long)((maxM + 31) / 32) * ((L.N + 31) / 32) <= 64;
 }
 
+// Whether a product that one 64 x 64 tile holds has its results over its own operands: its workgroup
+// has read them all before it stores the first result, several workgroups have not.
+bool one_tile_in_place(const Launch &L)
+{
+    if (L.N > 64 || L.epi == Epi::GLU) return false;
+    const size_t el = L.epi == Epi::I64 ? 8 : L.epi == Epi::F16 || L.epi == Epi::ACT || L.f16out ? 2 : 4;
+    for (int i = 0; i < L.nprob; i++) {
+        const Problem &P = L.prob[i];
+        if (P.M < 1 || P.M > 64) continue;
+        const uintptr_t c = (uintptr_t)P.C, c1 = c + (size_t)P.M * L.N * el;
+        const auto over = [&](const void *x, size_t bytes) { return (uintptr_t)x < c1 && c < (uintptr_t)x + bytes; };
+        if (over(P.A, (size_t)P.M * row_bytes(L.fmt_a, L.K)) || over(P.B, (size_t)L.N * row_bytes(L.fmt_b, L.K))) return true;
+    }
+    return false;
+}
+
 // [slice][M][N] planes of fp32 partials
 size_t ws_bytes_of(const Plan &p)
 {
@@ -685,7 +701,8 @@ hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
     }
     if (maxM == 0) return hipSuccess;
 
-    if (stream_takes(L, maxM)) {   // at most 16 rows
+    const bool in_place = !L.qa && one_tile_in_place(L);
+    if (!in_place && stream_takes(L, maxM)) {   // at most 16 rows
         uint64_t blocks = 0;
         const hipError_t e = stream_launch(L, &blocks);
         if (blocks_out) *blocks_out = blocks;
@@ -693,20 +710,20 @@ hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
     }
 
     if (L.qa && !stream_gw_takes(L, maxM)) return hipErrorInvalidValue;
-    if (stream_gw_takes(L, maxM)) {   // at most 16 rows, group-wise
+    if (!in_place && stream_gw_takes(L, maxM)) {   // at most 16 rows, group-wise
         uint64_t blocks = 0;
         const hipError_t e = stream_gw_launch(L, maxM, &blocks);
         if (blocks_out) *blocks_out = blocks;
         return e;
     }
 
-    if (mid_gw_takes(L, maxM)) {   // 17 rows and more, group-wise, as long as the workgroups fit the GPU
+    if (!in_place && mid_gw_takes(L, maxM)) {   // 17 rows and more, group-wise, as long as the workgroups fit the GPU
         uint64_t blocks = 0;
         const hipError_t e = mid_gw_launch(L, maxM, &blocks);
         if (blocks_out) *blocks_out = blocks;
         return e;
     }
-    if (small_takes(L, maxM)) {
+    if (!in_place && small_takes(L, maxM)) {
         const Problem &P = L.prob[0];
         const int nbm = (P.M + 31) / 32, nbn = (L.N + 31) / 32;
         const auto *A = static_cast<const _Float16 *>(P.A), *B = static_cast<const _Float16 *>(P.B);
@@ -718,7 +735,7 @@ hipError_t gemm_launch(const Launch &L, uint64_t *blocks_out)
         return hipGetLastError();
     }
 
-    Plan pl = plan_of(L, maxM, true);
+    Plan pl = plan_of(L, maxM, !in_place);
     if (pl.planes && (!L.ws || L.ws_bytes < ws_bytes_of(pl)))
         pl = plan_of(L, maxM, false);   // no workspace: the best plan with one slice per tile
     const int bm = pl.bm, bn = pl.bn;

@@ -277,6 +277,12 @@ static void routes()
     CHECK(fa(1, 8192, 256, 64, 32) && ran("k_fa_rows"));
     CHECK(fa(1, 8192, 256, 24, 24) && ran("k_fa_rows"));
     CHECK(fa(1, 8192, 64, 32, 32) && ran("k_fa_rows"));
+    // results over their own operands: one workgroup, which has read all of them first
+    CHECK(int8(4, 512, 64) && ran("k_stream"));
+    CHECK(rocket_matmul_int8(fd, 4, 512, 64, A, B, reinterpret_cast<int32_t *>(A)) == 0 && ran("k_gemm"));
+    CHECK(rocket_matmul_int8_groupwise(fd, 4, 512, 64, A, B, Y, W, reinterpret_cast<float *>(A), 64) == 0 && ran("k_gemm"));
+    CHECK(rocket_matmul_int8_groupwise(fd, 20, 512, 64, A, B, Y, W, reinterpret_cast<float *>(B), 64) == 0 && ran("k_gemm"));
+    CHECK(rocket_matmul_fp16(fd, 4, 1024, 64, h(X), h(W), h(X)) == 0 && ran("k_gemm"));
     // fp16, 17 to 32 rows of short K
     CHECK(fp16(fd, 32, 992, 32768) == 0 && ran("k_small_f16"));
     CHECK(fp16(fd, 32, 992, 65536) == 0 && ran("k_gemm"));

@@ -114,3 +114,48 @@ def test_capture_on_a_fresh_handle(lib, orc, monkeypatch, op):
     del g
     lib.rocket_close(warm)
     lib.rocket_close(fd)
+
+
+@pytest.mark.parametrize("M,K,N", [(4, 512, 64), (16, 992, 32), (20, 1024, 64), (64, 512, 64)])
+def test_one_tile_in_place(lib, orc, M, K, N):
+    """Products that one 64 x 64 tile holds, with their results over their own rows or weights: int8,
+    group-wise (int8 with scales per row), fp16 and bf16."""
+    import torch
+    print(f"one tile in place M={M} K={K} N={N}", flush=True)
+    N64 = (N + 63) // 64 * 64
+    A, B = orc.gen_i8((M, K), SEED + 20), orc.gen_i8((N64, K), SEED + 21)
+    rs, bs = orc.gen_uniform((M,), SEED + 22, 0.5, 1.5), orc.gen_uniform((N64, K // 32), SEED + 23, 0.005, 0.02)
+    x, W = orc.gen_normal((M, K), SEED + 24), orc.gen_normal((N, K), SEED + 25, 0, 0.02)
+    x16, W16 = (orc.f32_to_f16_bits(v).view(np.float16) for v in (x, W))
+    fd, ctx = lib.rocket_open(), lib.rocket_i8_ctx_create(1)
+    stream = torch.cuda.Stream()
+    for f in (fd, lib.rocket_i8_ctx_fd(ctx)):
+        _handle(lib, f, stream)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)  # noqa: E731
+    with torch.cuda.stream(stream):
+        if N == N64:
+            for over in (0, 1):
+                a, b = dev(A), dev(B)
+                c = (a, b)[over]
+                if c.numel() < M * N * 4:
+                    continue
+                assert lib.rocket_matmul_int8(fd, M, K, N, R.ptr(a), R.ptr(b), R.ptr(c)) == 0
+                got = c.flatten()[:M * N * 4].cpu().numpy().view(np.int32).reshape(M, N)
+                assert np.array_equal(got, orc.matmul_int8(A, B))
+            w = lib.rocket_i8_weights_pack_gw(ctx, M, K, N, R.ptr(B), 32)
+            a, r, s = dev(A), dev(rs), dev(bs)
+            if M * K >= M * N * 4:
+                assert lib.rocket_matmul_int8_prepacked_gw_rowscale(ctx, M, K, N, R.ptr(a), R.ptr(r), R.ptr(s), R.ptr(a), w) == 0
+                got = a.flatten()[:M * N * 4].cpu().numpy().view(np.float32).reshape(M, N)
+                assert np.array_equal(got, orc.matmul_gw_rowscale_f32(A, B, rs, bs, 32))
+            lib.rocket_i8_weights_free(ctx, w)
+        a, b = dev(x16), dev(W16)
+        assert lib.rocket_matmul_fp16(fd, M, K, N, R.ptr(a), R.ptr(b), R.ptr(a)) == 0
+        got = a.flatten()[:M * N].cpu().numpy().astype(np.float32).reshape(M, N)
+        want = orc.matmul_fp16_f32out(x16.view(np.uint16), W16.view(np.uint16))
+        assert orc.norm_err(got, want) < 1e-3        # rounded to fp16
+        a, b = dev(x), dev(W)
+        assert lib.rocket_matmul_bf16(fd, M, K, N, R.ptr(a), R.ptr(b), R.ptr(a)) == 0
+        assert orc.norm_err(a.flatten()[:M * N].cpu().numpy().reshape(M, N), orc.matmul_bf16(x, W)) < 1e-5
+    lib.rocket_i8_ctx_free(ctx)
+    lib.rocket_close(fd)
