@@ -48,7 +48,9 @@ int fa_gpu(int fd, const char *who, int T, int n_kv, int dk, int dv, int n_head,
     // they, and the mask's rows, are padded to a multiple of 64 keys (zeros), so that the mask's
     // tiles too go by DMA (64 x 3001 keys, heads of 256: 46.0 us with a padding copy of a thread a
     // value and the mask in 2-byte loads, 40.7 with eight values a thread, 28.2 with the mask too)
-    const int n_kvp = flash_attn_few_rows(f) || n_kv % 8 == 0 ? n_kv : round_up(n_kv, 64);
+    // (and where results lie over V, whose heads other workgroups may still read)
+    const bool over_v = (uintptr_t)out < (uintptr_t)V + h16(nv) && (uintptr_t)V < (uintptr_t)out + h16(no);
+    const int n_kvp = !over_v && (flash_attn_few_rows(f) || n_kv % 8 == 0) ? n_kv : round_up(n_kv, 64);
     const bool pad = n_kvp != n_kv;
     f.scale = scale; f.softcap = softcap;
     Call c(L.h, who);

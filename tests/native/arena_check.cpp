@@ -283,6 +283,9 @@ static void routes()
     CHECK(rocket_matmul_int8_groupwise(fd, 4, 512, 64, A, B, Y, W, reinterpret_cast<float *>(A), 64) == 0 && ran("k_gemm"));
     CHECK(rocket_matmul_int8_groupwise(fd, 20, 512, 64, A, B, Y, W, reinterpret_cast<float *>(B), 64) == 0 && ran("k_gemm"));
     CHECK(rocket_matmul_fp16(fd, 4, 1024, 64, h(X), h(W), h(X)) == 0 && ran("k_gemm"));
+    // attention's results over V: V is copied first where its rows are no multiple of a tile
+    CHECK(fa(1, 100, 64, 8, 8) && !ran("k_pad_cols"));
+    CHECK(rocket_flash_attn_fp16(fd, 1, 100, 64, 64, 8, 8, 0.1f, 0.f, h(X), h(W), h(Y), nullptr, h(Y)) == 0 && ran("k_pad_cols"));
     // fp16, 17 to 32 rows of short K
     CHECK(fp16(fd, 32, 992, 32768) == 0 && ran("k_small_f16"));
     CHECK(fp16(fd, 32, 992, 65536) == 0 && ran("k_gemm"));
