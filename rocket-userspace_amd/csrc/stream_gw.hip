@@ -46,6 +46,10 @@ struct GArgs {
     const void *A[kMaxProblems], *A2[kMaxProblems], *B[kMaxProblems];
     const float *as[kMaxProblems], *bs[kMaxProblems];
     void *C[kMaxProblems];
+};
+
+// A dumping launch's arguments (of their own: longer ones cost the other launches microseconds when cold).
+struct GArgsDump : GArgs {
     FewDump dump[kMaxProblems];
 };
 
@@ -73,7 +77,7 @@ __device__ __forceinline__ long lo64(i32x4 v) { return (long)(((unsigned long)(u
 // workgroup quantises by k_quant_rows' formula (act(A) * A2 where A2 is given). DUMP: the partials of
 // the launch's dump windows are stored too (an instantiation of its own: the stores cost registers).
 template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT, bool DUMP>
-__global__ __launch_bounds__(512, 2) void k_stream_gw(const GArgs a)
+__global__ __launch_bounds__(512, 2) void k_stream_gw(const std::conditional_t<DUMP, GArgsDump, GArgs> a)
 {
     constexpr bool I4 = FB == Fmt::I4P;
     constexpr int SK = I4 ? 128 : 64, NP = SK / PK;       // K elements and pieces a step
@@ -270,7 +274,8 @@ __global__ __launch_bounds__(512, 2) void k_stream_gw(const GArgs a)
     const char *const la = codes + am * kp;
     int slot = 0;
     const int npc = K / PK;    // pieces in all
-    [[maybe_unused]] const FewDump dw = a.dump[p];
+    [[maybe_unused]] FewDump dw = {};
+    if constexpr (DUMP) dw = a.dump[p];
     for (int sl = sl0; sl < sl1; sl++) {
         wait_vm_le(min(max(PRE, min(depth, own)) - 1, max(PRE, own) - 1 - (sl - sl0)) * kCH);
         asm volatile("" ::: "memory");   // no read of the slot above the wait
@@ -458,7 +463,7 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
     return !L.qa || (long)maxM * L.K <= 120L * g.w * 64;
 }
 
-template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT, bool DUMP> hipError_t launch_s(const GArgs &a, const GPlan &g, hipStream_t s)
+template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT, bool DUMP> hipError_t launch_s(const GArgsDump &a, const GPlan &g, hipStream_t s)
 {
     auto kern = k_stream_gw<FB, PK, PPG, RS, QIN, SPLIT, DUMP>;
     // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any thread
@@ -473,11 +478,12 @@ template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT, bool DUMP> hipE
             return hipGetLastError();
         opted.fetch_or(bit, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)(SPLIT ? a.nbn : (a.nbn + g.w - 1) / g.w), (unsigned)g.np), dim3(g.w * 64), g.lds, s, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(SPLIT ? a.nbn : (a.nbn + g.w - 1) / g.w), (unsigned)g.np), dim3(g.w * 64), g.lds, s,
+                       static_cast<const std::conditional_t<DUMP, GArgsDump, GArgs> &>(a));
     return hipGetLastError();
 }
 
-template <Fmt FB, int PK, int PPG, bool RS, int QIN> hipError_t launch_k(const GArgs &a, const GPlan &g, hipStream_t s)
+template <Fmt FB, int PK, int PPG, bool RS, int QIN> hipError_t launch_k(const GArgsDump &a, const GPlan &g, hipStream_t s)
 {
     if constexpr (QIN == 0)
         if (g.dump) {
@@ -490,7 +496,7 @@ template <Fmt FB, int PK, int PPG, bool RS, int QIN> hipError_t launch_k(const G
     return launch_s<FB, PK, PPG, RS, QIN, false, false>(a, g, s);
 }
 
-template <Fmt FB, int PK, int PPG> hipError_t launch_q(const GArgs &a, const GPlan &g, bool rs, int qa, hipStream_t s)
+template <Fmt FB, int PK, int PPG> hipError_t launch_q(const GArgsDump &a, const GPlan &g, bool rs, int qa, hipStream_t s)
 {
     if (!rs) return launch_k<FB, PK, PPG, false, 0>(a, g, s);
     if (qa == 1) return launch_k<FB, PK, PPG, true, 1>(a, g, s);
@@ -499,7 +505,7 @@ template <Fmt FB, int PK, int PPG> hipError_t launch_q(const GArgs &a, const GPl
     return qa ? hipErrorInvalidValue : launch_k<FB, PK, PPG, true, 0>(a, g, s);
 }
 
-template <Fmt FB, int PK> hipError_t launch_pk(const GArgs &a, const GPlan &g, const Launch &L)
+template <Fmt FB, int PK> hipError_t launch_pk(const GArgsDump &a, const GPlan &g, const Launch &L)
 {
     const bool rs = L.rowscale != 0;
     if (a.ppg == 1) return launch_q<FB, PK, 1>(a, g, rs, L.qa, L.stream);
@@ -519,7 +525,7 @@ bool stream_gw_takes(const Launch &L, int maxM)
 hipError_t stream_gw_launch(const Launch &L, int maxM, uint64_t *blocks)
 {
     GPlan g;
-    GArgs a = {};
+    GArgsDump a = {};
     if (!plan_gw(L, maxM, g, a)) return hipErrorInvalidValue;
     a.N = L.N;
     a.K = L.K;

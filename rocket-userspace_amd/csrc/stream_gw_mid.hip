@@ -31,6 +31,10 @@ struct MArgs {
     const void *A[kMaxProblems], *B[kMaxProblems];
     const float *as[kMaxProblems], *bs[kMaxProblems];
     void *C[kMaxProblems];
+};
+
+// A dumping launch's arguments (as in stream_gw.hip).
+struct MArgsDump : MArgs {
     FewDump dump[kMaxProblems];
 };
 
@@ -40,7 +44,7 @@ __device__ __forceinline__ long pair64(int a, int b) { return (long)(((unsigned 
 // groups a chunk). RS: a scale a row. MB: 16-row blocks a workgroup. Two or four waves. DUMP: the
 // partials of the launch's dump windows are stored too.
 template <Fmt FB, int PK, int PPG, bool RS, int MB, bool DUMP>
-__global__ __launch_bounds__(256, 2) void k_mid_gw(const MArgs a)
+__global__ __launch_bounds__(256, 2) void k_mid_gw(const std::conditional_t<DUMP, MArgsDump, MArgs> a)
 {
     constexpr bool I4 = FB == Fmt::I4P;
     // K elements and pieces a step; code bytes of a row and chunk
@@ -145,7 +149,8 @@ __global__ __launch_bounds__(256, 2) void k_mid_gw(const MArgs a)
     i32x4 d[MB];
 #pragma unroll
     for (int i = 0; i < MB; i++) acc[i] = f32x4{};
-    [[maybe_unused]] const FewDump dw = a.dump[p];
+    [[maybe_unused]] FewDump dw = {};
+    if constexpr (DUMP) dw = a.dump[p];
     for (int ch = 0; ch < nch; ch++) {
         // chunk ch has arrived (only the next chunk's instructions are outstanding; none once nothing more
         // was issued), in every wave after the barrier; every wave has read chunk ch - 1, whose place
@@ -296,7 +301,7 @@ bool plan_mid(const Launch &L, int maxM, MPlan &g, MArgs &a)
     return false;
 }
 
-template <Fmt FB, int PK, int PPG, bool RS, int MB, bool DUMP> hipError_t launch_mid_k(const MArgs &a, const MPlan &g, hipStream_t s)
+template <Fmt FB, int PK, int PPG, bool RS, int MB, bool DUMP> hipError_t launch_mid_k(const MArgsDump &a, const MPlan &g, hipStream_t s)
 {
     auto kern = k_mid_gw<FB, PK, PPG, RS, MB, DUMP>;
     // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any thread
@@ -311,11 +316,12 @@ template <Fmt FB, int PK, int PPG, bool RS, int MB, bool DUMP> hipError_t launch
             return hipGetLastError();
         opted.fetch_or(bit, std::memory_order_release);
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)((a.nbn + g.w - 1) / g.w), (unsigned)g.np, (unsigned)g.nb), dim3(g.w * 64), g.lds, s, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((a.nbn + g.w - 1) / g.w), (unsigned)g.np, (unsigned)g.nb), dim3(g.w * 64), g.lds, s,
+                       static_cast<const std::conditional_t<DUMP, MArgsDump, MArgs> &>(a));
     return hipGetLastError();
 }
 
-template <Fmt FB, int PK> hipError_t launch_mid_pk(const MArgs &a, const MPlan &g, const Launch &L)
+template <Fmt FB, int PK> hipError_t launch_mid_pk(const MArgsDump &a, const MPlan &g, const Launch &L)
 {
     auto by = [&](auto PPG, auto RS) {
         constexpr int P = decltype(PPG)::value;
@@ -343,7 +349,7 @@ bool mid_gw_takes(const Launch &L, int maxM)
 hipError_t mid_gw_launch(const Launch &L, int maxM, uint64_t *blocks)
 {
     MPlan g;
-    MArgs a = {};
+    MArgsDump a = {};
     if (!plan_mid(L, maxM, g, a)) return hipErrorInvalidValue;
     a.N = L.N;
     a.K = L.K;
