@@ -573,16 +573,16 @@ __global__ __launch_bounds__(256) void k_fa_combine(const void *__restrict__ par
 // Eight output columns a thread (cols_pad a multiple of 8, dst 16-byte aligned): one unaligned
 // 16-byte load, one aligned store (a thread a column took 13 us for 2048 rows of 3000).
 struct __attribute__((packed, aligned(2))) Halves8 { f16x8 v; };
-// Rows [0, rows) come from src, the next rows2 from src2 (one launch for V and the mask).
+// Rows [0, rows) come from src, the next rows2 from src2 (one launch for V and the mask). A
+// workgroup is 2^lx chunks of 256 >> lx rows: no division (one by a run-time row length a thread took a
+// quarter of a microsecond of short calls).
 __global__ __launch_bounds__(256) void k_pad_cols(const _Float16 *__restrict__ src, _Float16 *__restrict__ dst, long rows,
                                                   const _Float16 *__restrict__ src2, _Float16 *__restrict__ dst2, long rows2,
-                                                  int cols, int cols_pad)
+                                                  int cols, int cols_pad, int lx)
 {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int per = cols_pad / 8;
-    if (i >= (rows + rows2) * per) return;
-    long r = i / per;
-    const int c = (int)(i - r * per) * 8;
+    long r = ((long)blockIdx.x << (8 - lx)) + (threadIdx.x >> lx);
+    const int c = (int)((blockIdx.y << lx) + (threadIdx.x & ((1u << lx) - 1))) * 8;
+    if (c >= cols_pad || r >= rows + rows2) return;
     if (r >= rows) {
         r -= rows;
         src = src2;
@@ -590,8 +590,16 @@ __global__ __launch_bounds__(256) void k_pad_cols(const _Float16 *__restrict__ s
     }
     const _Float16 *row = src + r * cols;
     f16x8 v = {};
-    if (c + 8 <= cols) {
-        v = reinterpret_cast<const Halves8 *>(row + c)->v;
+    const int past = c + 8 - cols;   // columns past the row's end
+    if (cols >= 8) {
+        // one load either way: the row's last eight, shifted, where it ends inside
+        const f16x8 x = reinterpret_cast<const Halves8 *>(row + (past > 0 ? cols - 8 : c))->v;
+        unsigned long w[2];
+        __builtin_memcpy(w, &x, 16);
+        if (past >= 8) w[0] = w[1] = 0;
+        else if (past >= 4) w[0] = w[1] >> (16 * past - 64), w[1] = 0;
+        else if (past > 0) w[0] = w[0] >> (16 * past) | w[1] << (64 - 16 * past), w[1] >>= 16 * past;
+        __builtin_memcpy(&v, w, 16);
     } else {
 #pragma unroll
         for (int e = 0; e < 8; e++)
@@ -754,10 +762,12 @@ hipError_t pad_cols_f16(const _Float16 *src, _Float16 *dst, long rows, const _Fl
 {
     if (rows < 1 || rows2 < 0 || cols < 1 || cols_pad < cols || cols_pad % 8 || !al(dst, 16) || (rows2 && !al(dst2, 16)))
         return hipErrorInvalidValue;
-    const long n = (rows + rows2) * (cols_pad / 8), blocks = (n + 255) / 256;
-    if (blocks > 0x7FFFFFFFL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_pad_cols, dim3((unsigned)blocks), dim3(256), 0, s, src, dst, rows, src2, dst2, rows2, cols, cols_pad);
-    if (blocks_out) *blocks_out = (uint64_t)blocks;
+    int lx = 3;
+    while (lx < 8 && 8 << lx < cols_pad) lx++;
+    const long y = (cols_pad / 8 + (1 << lx) - 1) >> lx, x = (rows + rows2 + (256 >> lx) - 1) / (256 >> lx);
+    if (x > 0x7FFFFFL || y > 65535) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_pad_cols, dim3((unsigned)x, (unsigned)y), dim3(256), 0, s, src, dst, rows, src2, dst2, rows2, cols, cols_pad, lx);
+    if (blocks_out) *blocks_out = (uint64_t)(x * y);
     return hipGetLastError();
 }
 
