@@ -18,6 +18,7 @@
 // key order, so each V^T fragment is one 16-byte LDS read. O is rescaled only when some
 // running max grows by more than 8.
 #include "attn.h"
+#include "lds_optin.h"
 
 #include <atomic>
 #include <type_traits>
@@ -626,18 +627,8 @@ hipError_t launch_fa(const FaArgs &a, dim3 grid, hipStream_t s)
     constexpr int lds = CF::template lds<MVEC>();
     static_assert(lds <= 160 * 1024, "LDS budget");
     auto kern = k_flash_attn<DHP, DVP, MVEC, CAP>;
-    // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any
-    // thread may launch, so the mask is atomic)
     static std::atomic<uint64_t> opted{0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return hipGetLastError();
-    const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
-    if (!bit || !(opted.load(std::memory_order_acquire) & bit)) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                lds) != hipSuccess)
-            return hipGetLastError();
-        opted.fetch_or(bit, std::memory_order_release);
-    }
+    if (const hipError_t e = lds_opt_in(reinterpret_cast<const void *>(kern), lds, opted)) return e;
     hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, a);
     return hipGetLastError();
 }

@@ -20,6 +20,7 @@
 //   1 x 4096 keys, 32 / 8 heads of 128    16.8 ->  9.9
 //   8 x 3000 keys, 16 / 8 heads of 256    32.6 -> 13.4
 #include "attn.h"
+#include "lds_optin.h"
 
 #include <algorithm>
 #include <atomic>
@@ -296,18 +297,8 @@ template <int D, bool CAP, bool FULL> hipError_t launch_rows_f(const RowArgs &a,
     const int R = a.gqa * a.T;
     const size_t lds = (size_t)kWaves * R * ((D + 4) * 4 + 8);
     if (lds > 64 * 1024) {
-        // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any
-        // thread may launch, so the mask is atomic)
         static std::atomic<uint64_t> opted{0};
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return hipGetLastError();
-        const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
-        if (!bit || !(opted.load(std::memory_order_acquire) & bit)) {
-            if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    80 * 1024) != hipSuccess)
-                return hipGetLastError();
-            opted.fetch_or(bit, std::memory_order_release);
-        }
+        if (const hipError_t e = lds_opt_in(reinterpret_cast<const void *>(kern), 80 * 1024, opted)) return e;
     }
     hipLaunchKernelGGL(kern, dim3((unsigned)kv_heads, (unsigned)a.nsplit), dim3(kWaves * 64), lds, s, a);
     return hipGetLastError();

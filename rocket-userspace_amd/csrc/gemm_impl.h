@@ -29,6 +29,7 @@
 #pragma once
 
 #include "gemm.h"
+#include "lds_optin.h"
 
 #include <stdlib.h>
 
@@ -1817,18 +1818,8 @@ hipError_t launch_one(const KArgs &ka, int blocks, hipStream_t s)
     constexpr int lds = CF::ADMA ? CF::LDS_ADMA : CF::LDS_RING;
     static_assert(lds <= 160 * 1024, "LDS budget");
     auto kern = k_gemm<BM, BN, FA, FB, MATH, EPI, RS, GM>;
-    // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any
-    // thread may launch, so the mask is atomic)
     static std::atomic<uint64_t> opted{0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return hipGetLastError();
-    const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
-    if (!bit || !(opted.load(std::memory_order_acquire) & bit)) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                lds) != hipSuccess)
-            return hipGetLastError();
-        opted.fetch_or(bit, std::memory_order_release);
-    }
+    if (const hipError_t e = lds_opt_in(reinterpret_cast<const void *>(kern), lds, opted)) return e;
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(CF::NT), lds, s, ka);
     return hipGetLastError();
 }
@@ -1880,6 +1871,26 @@ hipError_t dispatch_bf16(int bm, int bn, const Launch &L, const KArgs &ka, int b
 
 // HBM bytes of one operand row of K elements.
 long row_bytes(Fmt f, int K);
+
+// Two words as the 64-bit operand of an 8-byte MFMA fragment.
+__device__ __forceinline__ long pair64(int a, int b) { return (long)(((unsigned long)(unsigned)b << 32) | (unsigned)a); }
+
+// The few-row group-wise kernels' table of a wave's b scales, S[group][16 columns]: lane (column r16,
+// quarter q) takes the groups 16 i + 4 q .. + 3 of its column, loaded (zeros past nG) and stored (int4
+// ones by 1/16: unpacked int4 carries x16).
+__device__ __forceinline__ void load_scales(Rsrc sb, int nG, int r16, int q, int i, float (&v)[4])
+{
+    const int g = 16 * i + 4 * q;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = ld4f(sb, g + e < nG ? (uint32_t)(r16 * nG + g + e) * 4u : kOOB);
+}
+template <bool I4> __device__ __forceinline__ void store_scales(float *S, int nGp, int r16, int q, int i, const float (&v)[4])
+{
+    const int g = 16 * i + 4 * q;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (g + e < nGp) S[(g + e) * 16 + r16] = I4 ? v[e] * 0.0625f : v[e];
+}
 
 // A dump window of a few-row launch's problem (Problem::dump and its rows, null: none), and the store of
 // group g's partials for column n: d[e] is row m + e, times 16 with packed int4 weights.

@@ -69,8 +69,6 @@ __device__ __forceinline__ void wait_vm_le(int n)
     else wait_vm<0>();
 }
 
-__device__ __forceinline__ long lo64(i32x4 v) { return (long)(((unsigned long)(unsigned)v[1] << 32) | (unsigned)v[0]); }
-
 // PK: K of an MFMA piece (32, 64 or, int4, 128), a divisor of the group; PPG: pieces a group (1 or
 // 2: whole groups a slot, so that a slot's body has no branch and its LDS reads, MFMAs and folds
 // overlap; 0: any number, counted). RS: a scale a row. QIN: 0 int8 codes in global memory, 1 / 2 fp32 / fp16 rows that each
@@ -112,17 +110,8 @@ __global__ __launch_bounds__(512, 2) void k_stream_gw(const std::conditional_t<D
     constexpr int SR = 4;   // in registers: 64 groups; further ones after the ring's first loads
     const int i0 = SPLIT ? wave : 0, di = SPLIT ? W : 1;
     float sv[SR][4];
-    auto sload = [&](int i, float (&v)[4]) __attribute__((always_inline)) {
-        const int g = 16 * i + 4 * q;
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = ld4f(sb, g + e < nG ? (uint32_t)(r16 * nG + g + e) * 4u : kOOB);
-    };
-    auto sstore = [&](int i, const float (&v)[4]) __attribute__((always_inline)) {
-        const int g = 16 * i + 4 * q;
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            if (g + e < nGp) S[(g + e) * 16 + r16] = I4 ? v[e] * 0.0625f : v[e];   // 1/16: unpacked int4 carries x16
-    };
+    auto sload = [&](int i, float (&v)[4]) __attribute__((always_inline)) { load_scales(sb, nG, r16, q, i, v); };
+    auto sstore = [&](int i, const float (&v)[4]) __attribute__((always_inline)) { store_scales<I4>(S, nGp, r16, q, i, v); };
 #pragma unroll
     for (int i = 0; i < SR; i++)
         if (16 * (i0 + i * di) < nGp) sload(i0 + i * di, sv[i]);
@@ -295,7 +284,7 @@ __global__ __launch_bounds__(512, 2) void k_stream_gw(const std::conditional_t<D
                     const long af = *reinterpret_cast<const long *>(la + (((c0 + 2 * x + (q >> 1)) ^ am) << 4) + 8 * (q & 1));
                     if constexpr (I4) {
                         const int w = *reinterpret_cast<const int *>(ws + (16 * x + r16) * 16 + 4 * q);
-                        d = __builtin_amdgcn_mfma_i32_16x16x32_i8(af, lo64(i32x4{nib_hi(w), nib_lo(w), 0, 0}), z, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_i32_16x16x32_i8(af, pair64(nib_hi(w), nib_lo(w)), z, 0, 0, 0);
                     } else {
                         const long w = *reinterpret_cast<const long *>(ws + (16 * (2 * x + (q >> 1)) + r16) * 16 + 8 * (q & 1));
                         d = __builtin_amdgcn_mfma_i32_16x16x32_i8(af, w, z, 0, 0, 0);
@@ -466,18 +455,8 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
 template <Fmt FB, int PK, int PPG, bool RS, int QIN, bool SPLIT, bool DUMP> hipError_t launch_s(const GArgsDump &a, const GPlan &g, hipStream_t s)
 {
     auto kern = k_stream_gw<FB, PK, PPG, RS, QIN, SPLIT, DUMP>;
-    // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any thread
-    // may launch, so the mask is atomic)
     static std::atomic<uint64_t> opted{0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return hipGetLastError();
-    const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
-    if (!bit || !(opted.load(std::memory_order_acquire) & bit)) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024) != hipSuccess)
-            return hipGetLastError();
-        opted.fetch_or(bit, std::memory_order_release);
-    }
+    if (const hipError_t e = lds_opt_in(reinterpret_cast<const void *>(kern), 160 * 1024, opted)) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)(SPLIT ? a.nbn : (a.nbn + g.w - 1) / g.w), (unsigned)g.np), dim3(g.w * 64), g.lds, s,
                        static_cast<const std::conditional_t<DUMP, GArgsDump, GArgs> &>(a));
     return hipGetLastError();

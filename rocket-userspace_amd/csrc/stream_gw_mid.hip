@@ -38,8 +38,6 @@ struct MArgsDump : MArgs {
     FewDump dump[kMaxProblems];
 };
 
-__device__ __forceinline__ long pair64(int a, int b) { return (long)(((unsigned long)(unsigned)b << 32) | (unsigned)a); }
-
 // PK: K of an MFMA piece (32, 64 or, int4, 128); a group is PPG pieces (1, or 2 of a whole step: whole
 // groups a chunk). RS: a scale a row. MB: 16-row blocks a workgroup. Two or four waves. DUMP: the
 // partials of the launch's dump windows are stored too.
@@ -71,17 +69,8 @@ __global__ __launch_bounds__(256, 2) void k_mid_gw(const std::conditional_t<DUMP
     const Rsrc sb = rsrc(a.bs[p] + (size_t)(live ? n0 : 0) * nG, live ? (uint32_t)(16 * nG) * 4u : 0u);
     constexpr int SR = 4;
     float sv[SR][4];
-    auto sload = [&](int i, float (&v)[4]) __attribute__((always_inline)) {
-        const int g = 16 * i + 4 * q;
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = ld4f(sb, g + e < nG ? (uint32_t)(r16 * nG + g + e) * 4u : kOOB);
-    };
-    auto sstore = [&](int i, const float (&v)[4]) __attribute__((always_inline)) {
-        const int g = 16 * i + 4 * q;
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            if (g + e < nGp) S[(g + e) * 16 + r16] = I4 ? v[e] * 0.0625f : v[e];   // 1/16: unpacked int4 carries x16
-    };
+    auto sload = [&](int i, float (&v)[4]) __attribute__((always_inline)) { load_scales(sb, nG, r16, q, i, v); };
+    auto sstore = [&](int i, const float (&v)[4]) __attribute__((always_inline)) { store_scales<I4>(S, nGp, r16, q, i, v); };
 #pragma unroll
     for (int i = 0; i < SR; i++)
         if (16 * i < nGp) sload(i, sv[i]);
@@ -304,18 +293,8 @@ bool plan_mid(const Launch &L, int maxM, MPlan &g, MArgs &a)
 template <Fmt FB, int PK, int PPG, bool RS, int MB, bool DUMP> hipError_t launch_mid_k(const MArgsDump &a, const MPlan &g, hipStream_t s)
 {
     auto kern = k_mid_gw<FB, PK, PPG, RS, MB, DUMP>;
-    // dynamic LDS above 64 KiB needs an opt-in, once per device (bit d of the mask; any thread
-    // may launch, so the mask is atomic)
     static std::atomic<uint64_t> opted{0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return hipGetLastError();
-    const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
-    if (!bit || !(opted.load(std::memory_order_acquire) & bit)) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                160 * 1024) != hipSuccess)
-            return hipGetLastError();
-        opted.fetch_or(bit, std::memory_order_release);
-    }
+    if (const hipError_t e = lds_opt_in(reinterpret_cast<const void *>(kern), 160 * 1024, opted)) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)((a.nbn + g.w - 1) / g.w), (unsigned)g.np, (unsigned)g.nb), dim3(g.w * 64), g.lds, s,
                        static_cast<const std::conditional_t<DUMP, MArgsDump, MArgs> &>(a));
     return hipGetLastError();
