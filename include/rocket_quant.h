@@ -35,8 +35,11 @@ int rocket_quantize_rows_int8_fp16(int fd, int M, int K, const _Float16 *A, int8
 /* The resident group-wise products on fp32 activations: A is quantised per row into the
  * handle's arena by the pre-pass above, then the *_rowscale kernel runs with those codes and
  * scales — the same bits as rocket_quantize_rows_int8 followed by
- * rocket_matmul_int{8,4}_prepacked_gw_rowscale, in one call (two launches, or one that also quantises for few rows; the int8 codes
- * never leave the GPU). Same checks and return codes as the *_rowscale entry each mirrors. */
+ * rocket_matmul_int{8,4}_prepacked_gw_rowscale, in one call (the int8 codes never leave the GPU).
+ * Two launches; one, whose product quantises the rows itself, for few rows of moderate K (up to 16
+ * rows and about 61440 elements in all, fewer where a workgroup has fewer waves or its LDS does not
+ * hold them, and results not stored over the rows). This holds for every entry below that quantises.
+ * Same checks and return codes as the *_rowscale entry each mirrors. */
 int rocket_matmul_int8_prepacked_gw_f32in(rocket_i8_ctx *ctx, int M, int K, int N, const float *A,
                                           const float *b_scale, float *Cf, rocket_i8_weights *w);
 int rocket_matmul_int4_prepacked_gw_f32in(rocket_i4_ctx *ctx, int M, int K, int N, const float *A,

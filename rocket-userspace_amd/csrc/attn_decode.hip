@@ -13,12 +13,12 @@
 // holds query l % 16. The 16 rows of K block b are keys 8 (i / 4) + 4 b + i % 4, so that lane
 // quarter q ends up with keys 8 q .. 8 q + 7 of the chunk, which is what the second product's
 // operand takes: O^T += V^T P^T, P rounded to fp16 in registers. The waves' outputs merge in
-// LDS, the workgroups' in k_fa_merge.
+// LDS, the workgroups' in k_fa_merge; a short cache is one workgroup's, and has no merge.
 //
-// Measured (three sets of operands in turn; before, with attn.hip; after):
-//   1 x 3000 keys, 16 / 8 heads of 256    31.7 -> 11.4 us  (24.6 MB of K and V; 7.4 us the kernel, 3.3 TB/s)
-//   1 x 4096 keys, 32 / 8 heads of 128    16.8 ->  9.9
-//   8 x 3000 keys, 16 / 8 heads of 256    32.6 -> 13.4
+// Measured (sets of operands in turn; before, with attn.hip; after):
+//   1 x 3000 keys, 16 / 8 heads of 256    31.6 -> 10.8 us  (24.6 MB of K and V; 8.0 us the kernel, 3.1 TB/s)
+//   1 x 4096 keys, 32 / 8 heads of 128    18.2 ->  8.8
+//   8 x 3000 keys, 16 / 8 heads of 256    33.5 -> 14.2     (with a mask)
 #include "attn.h"
 #include "lds_optin.h"
 
@@ -84,9 +84,9 @@ __device__ __forceinline__ i32x4 row8(const _Float16 *row, int key, int n)
 
 // Merges the splits, one (head, token) row a workgroup: out = sum_s w_s On_s / sum_s w_s with
 // w_s = 2^(m_s - m) l_s, for up to 64 splits. The outputs are fp32, as one workgroup without splits
-// holds them: caches from a few hundred keys on are split here, and a rounding of each split's output
-// to fp16 beside those of the probabilities and of the result would cost a fifth more error (192 to
-// 448 keys, heads of 256: 2.8e-4 of the result, with it 3.4e-4). The splits spread over
+// holds them: caches from 257 keys on are split here, and a rounding of each split's output to fp16
+// beside those of the probabilities and of the result would cost a quarter more error (448 keys, heads
+// of 256: 2.5e-4 of the result, with it 3.2e-4). The splits spread over
 // the workgroup's 256 threads (dv / 8 threads a split), whose sums add in LDS. (A merge by each KV
 // head's last workgroup instead of this launch, on an arrival counter, measured 15.5 against 11.1
 // us at 3000 keys: the counter's release and acquire write back and invalidate the XCD's L2, and

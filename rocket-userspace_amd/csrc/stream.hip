@@ -1,4 +1,5 @@
-// stream.hip — products of at most 16 rows (decode batches): the weight-streaming kernels.
+// stream.hip — products of at most 16 rows, plain fp16 up to 32 (decode batches): the weight-streaming
+// kernels.
 //
 // With so few activation rows a product reads every weight once and does little with it: what
 // bounds it is how many bytes of B are in flight. The tiled kernels (gemm_impl.h) walk K in LDS
@@ -18,7 +19,7 @@
 //   tf32     4 x  4096 x  4096   46.8 -> 13.4 us
 //   FFN      1 x  3840 x 15360  118.3 -> 68.0 us   (two launches, 5.2 TB/s)
 // A copy of 4 GB runs at 4.9 TB/s (read + write). At 32 rows the activations' own fragments
-// are twice the bytes of B's through each CU's L1, and the tiled kernels in K slices win
+// are twice the bytes of B's through each CU's L1, and the tiled kernels win over k_stream
 // (fp16 32 x 3840 x 15360: 55.5 us here, 34.3 there). B loaded non-temporally was slower
 // throughout (the FFN at one row 68 -> 86 us).
 #include "gemm_impl.h"
@@ -300,9 +301,11 @@ hipError_t launch_chain(SArgs &a, const Launch &L, uint64_t *blocks)
 template <Fmt FA, Fmt FB, int KS> hipError_t launch_ks(SArgs &a, const Launch &L, uint64_t *blocks)
 {
     a.per = (a.nsteps + KS - 1) / KS;
-    // 32 columns a workgroup (the activations' fragments shared by two column blocks) where N
-    // gives every CU one and a half of them: fp16 16 x 3840 x 15360 38.5 -> 31.3 us, 4 rows 27.0
-    // -> 26.0; at N = 8192, one workgroup a CU, it loses (16 x 4096 x 8192 16.6 -> 18.8 us)
+    // 32 columns a workgroup (the activations' fragments shared by two column blocks) from one and a half
+    // of them a CU. K = 3840, N = 15360: int4 16 rows 12.2 -> 9.5 us, 4 rows 8.5 -> 8.0; bf16 65.7 ->
+    // 52.9 and 47.0 -> 43.7; tf32, whose splitting it does not share, 66.4 -> 65.6 and 47.5 -> 61.0. At
+    // N = 4096, half a workgroup a CU, it loses: int4 4.9 -> 5.7 and 3.9 -> 4.9, bf16 16.1 -> 22.5 and
+    // 13.0 -> 19.0. (N = 8192 and 12288 go either way, 0.86 to 1.25 times.)
     const bool glu = L.epi == Epi::GLU, wide = !glu && a.N >= 12288;
     const dim3 grid((unsigned)((a.N + (wide ? 31 : 15)) / (wide ? 32 : 16)), (unsigned)L.nprob);
     *blocks = (uint64_t)grid.x * grid.y;
@@ -322,7 +325,7 @@ template <Fmt FA, Fmt FB> hipError_t launch_fmt(SArgs &a, const Launch &L, uint6
     // Sixteen K slices where a wave's slice then still spans four sets of loads: the fp32
     // operands from K = 8192 (tf32 4 x 8192 x 4096 40.1 -> 31.7 us; at K = 4096 they lose, 13.4 ->
     // 16.2) and the gated pair from K = 2048 (K = 3840, with the down product 71.1 -> 68.0 us).
-    // Else eight: fp16 4 x 8192 x 4096 takes 12.9 us with eight and 15.8 with sixteen.
+    // Else eight: fp16 4 x 8192 x 4096 (a block's second product) 12.9 us with eight, 15.8 with sixteen.
     constexpr bool F32 = FA == Fmt::F32BF16 || FA == Fmt::F32TF32 || FB == Fmt::F32BF16 || FB == Fmt::F32TF32 || FB == Fmt::BF16X2 ||
                          FB == Fmt::BF16;
     if constexpr (F32 || FA == Fmt::F16)

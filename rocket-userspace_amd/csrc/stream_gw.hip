@@ -16,7 +16,7 @@
 //   int4 g 128   4 x  3840 x 15360   22.7 -> 10.6 us   (29.5 MB of codes, 3.0 TB/s)
 //   the same on fp32 rows             25.8 -> 11.5      (quantised in the kernel)
 //   int4 g 128   4 x  4096 x  4096   19.1 ->  6.0
-//   int4 g 32    4 x  4096 x  4096   27.9 -> 10.6
+//   int4 g 32    4 x  4096 x  4096   27.9 ->  9.5
 //   MoE layer, 16 tokens, g 32       35.0 -> 27.9      (two launches instead of three)
 // Other forms measured at 4 x 3840 x 15360: fragments through registers, partials exchanged in
 // LDS by rounds with a barrier each, 11.8 us (MoE 33); the same with a persistent grid 14.5, and

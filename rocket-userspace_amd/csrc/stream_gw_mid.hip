@@ -10,7 +10,7 @@
 // What bounds it is the serial time of a chunk (barrier, LDS reads, MFMA chain, fold) and a CU's
 // load rate, not HBM. The tiled kernel's stage is 0.75 us for the same 128 of K whatever M; here
 // (W4A8, rows quantised ahead, before -> after): 32 x 4096 x 4096 groups of 128 20.1 -> 9.9 us,
-// 128 x 2048 x 2048 14.9 -> 9.1, 256 x 7936 x 1024 34.4 -> 16.5, 64 x 3840 x 15360 25.3 -> 15.6.
+// 128 x 2048 x 2048 12.4 -> 6.7, 256 x 7936 x 1024 34.4 -> 16.5, 64 x 3840 x 15360 25.3 -> 15.6.
 #include "gemm_impl.h"
 
 namespace rk {
