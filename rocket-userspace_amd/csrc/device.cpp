@@ -14,6 +14,7 @@
 
 #include <atomic>
 #include <chrono>
+#include <new>
 #include <thread>
 
 namespace rk {
@@ -247,8 +248,15 @@ int Call::begin()
     }
     if (need_ + opt_ > h_->arena_cap) {
         if (hipStreamSynchronize(h_->stream) != hipSuccess) { (void)hipGetLastError(); return err_ = ROCKET_E_DEVICE; }
-        if (h_->arena_held) h_->retired.push_back(h_->arena);
-        else dev_free(h_->arena);
+        if (h_->arena_held) {
+            try {
+                h_->retired.push_back(h_->arena);
+            } catch (const std::bad_alloc &) {
+                return err_ = ROCKET_E_NOMEM;   // (the graph's arena stays the handle's)
+            }
+        } else {
+            dev_free(h_->arena);
+        }
         h_->arena_held = false;
         h_->arena = nullptr;
         h_->arena_cap = 0;

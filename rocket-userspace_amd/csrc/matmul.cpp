@@ -12,6 +12,8 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
+#include <new>
 #include <vector>
 
 namespace rk {
@@ -79,11 +81,11 @@ bool results_overlap_rows(const Req &r, size_t a_row, size_t c_elem)
     };
     constexpr int kFew = 24;
     Range few[kFew];
-    std::vector<Range> many;
+    std::unique_ptr<Range[]> many;
     Range *v = few;
     if (r.nprob > kFew / 3) {
-        many.resize((size_t)r.nprob * 3);
-        v = many.data();
+        many.reset(new (std::nothrow) Range[(size_t)r.nprob * 3]);
+        if (!(v = many.get())) return true;   // (no host memory: as if they did, which is right for all)
     }
     size_t n = 0;
     for (int p = 0; p < r.nprob; p++) {

@@ -6,8 +6,11 @@
 
 #include <stdio.h>
 
+#include <stdlib.h>
+
 #include <algorithm>
 #include <chrono>
+#include <new>
 #include <random>
 
 #include "ops.h"
@@ -16,6 +19,22 @@
 #include "rocket_hip.h"
 #include "rocket_matmul.h"
 #include "rocket_npu.h"
+
+// Host allocations of at least g_refuse bytes fail (0: none does).
+static size_t g_refuse = 0;
+void *operator new(size_t n)
+{
+    void *const p = g_refuse && n >= g_refuse ? nullptr : malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void *operator new(size_t n, const std::nothrow_t &) noexcept { return g_refuse && n >= g_refuse ? nullptr : malloc(n ? n : 1); }
+void *operator new[](size_t n) { return operator new(n); }
+void *operator new[](size_t n, const std::nothrow_t &t) noexcept { return operator new(n, t); }
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+void operator delete[](void *p) noexcept { free(p); }
+void operator delete[](void *p, size_t) noexcept { free(p); }
 
 static int g_fail = 0;
 #define CHECK(c)                                                                                       \
@@ -292,6 +311,48 @@ static void routes()
     rocket_close(fd);
 }
 
+// No host memory for the lists that a growing arena and the overlap check keep: an error code, or the
+// answer that is right for all; no exception leaves a C entry.
+static void short_of_host_memory()
+{
+    auto &f = fake::st();
+    const int fd = open_async();
+    CHECK(bf16(fd, 128, 8192, 512) == 0);
+    captured([&] { return bf16(fd, 128, 8192, 512); });
+    const int frees = f.frees;
+    g_refuse = 1;
+    int rc = 1;
+    try {
+        rc = rocket_matmul_bf16(fd, 512, 8192, 512, X, W, Y);
+    } catch (...) {
+    }
+    g_refuse = 0;
+    CHECK(rc == ROCKET_E_NOMEM);
+    CHECK(f.frees == frees);
+    CHECK(bf16(fd, 512, 8192, 512) == 0);
+    CHECK(f.frees == frees);
+    rocket_close(fd);
+
+    std::vector<int> M(64, 4);
+    std::vector<const void *> A(64, X);
+    std::vector<void *> C(64, Y);
+    rk::Req r;
+    r.nprob = 64;
+    r.M = M.data();
+    r.A = A.data();
+    r.C = C.data();
+    r.N = 64;
+    CHECK(!rk::results_overlap_rows(r, 64, 4));
+    g_refuse = 1;
+    bool over = false;
+    try {
+        over = rk::results_overlap_rows(r, 64, 4);
+    } catch (...) {
+    }
+    g_refuse = 0;
+    CHECK(over);
+}
+
 int main()
 {
     arena_kept_for_graphs();
@@ -301,6 +362,7 @@ int main()
     dumps_run_the_same_kernel();
     overlaps();
     routes();
+    short_of_host_memory();
     if (g_fail) {
         fprintf(stderr, "arena_check: %d check(s) failed\n", g_fail);
         return 1;
