@@ -274,7 +274,7 @@ bool plan_mid(const Launch &L, int maxM, MPlan &g, MArgs &a)
     static const int form[][2] = {{1, 1}, {2, 1}, {2, 2}};
     for (const auto &f : form) {
         if (f[1] == 2 && !i4 && L.group < 64) continue;
-        if (!i4 && L.K > 2048 && ((f[1] == 2 && maxM > 32) || (f[0] == 2 && L.group < 64 && L.N >= 8192))) continue;
+        if (!i4 && L.K >= 2048 && ((f[1] == 2 && maxM > 32) || (f[0] == 2 && L.group < 64 && L.N >= 8192))) continue;
         g.mb = f[0];
         const int chunk = sk * mid_steps(g.mb);
         a.nch = (L.K + chunk - 1) / chunk;

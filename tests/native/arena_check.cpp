@@ -268,7 +268,9 @@ static void routes()
     CHECK(gw8(16, 8192, 16384, 32) && ran("k_gemm"));
     CHECK(gw8(16, 8192, 8192, 64) && ran("k_gemm"));
     // int8 weights, 17 rows and more, long rows
-    CHECK(gw8(64, 2048, 16384, 64) && ran("k_mid_gw"));
+    CHECK(gw8(64, 1024, 16384, 64) && ran("k_mid_gw"));
+    CHECK(gw8(64, 2048, 16384, 64) && ran("k_gemm"));
+    CHECK(gw8(64, 2048, 8192, 32) && ran("k_gemm"));
     CHECK(gw8(64, 8192, 16384, 64) && ran("k_gemm"));
     CHECK(gw8(48, 8192, 6144, 32) && ran("k_mid_gw"));
     CHECK(gw8(48, 8192, 8192, 32) && ran("k_gemm"));
