@@ -290,10 +290,12 @@ hipError_t launch_chain(SArgs &a, const Launch &L, uint64_t *blocks)
     using I2 = std::integral_constant<int, 2>;
     using I5 = std::integral_constant<int, 5>;
     using I7 = std::integral_constant<int, 7>;
-    // two column blocks a wave share the rows' fragments where the columns still give a CU two waves
-    // (16 x 3072 x 16384 23.6 -> 19.8 us; 16 x 4096 x 8192 17.2 and 18.5)
+    // two column blocks a wave share the rows' fragments where the columns still give a CU one and a half
+    // waves (16 x 3072 x 16384 23.6 -> 19.8 us; 16 x 4096 x 8192 17.2 and 18.5), but for rows of 8 KB, of
+    // which 32 at a time meet in the same channels (16 x 4096 x 16384: two 38.0, one 31.4; 16 x 4096 x 40960
+    // 1.09 of the tiles' rate with one, 1.31 with two)
     if (maxM > 16) go(I2{}, I1{}, I5{});
-    else if (maxM > 4 && a.N >= 16384) go(I1{}, I2{}, I5{});
+    else if (maxM > 4 && a.N > 12288 && (a.ldb != 8192 || a.N > 20480)) go(I1{}, I2{}, I5{});
     else go(I1{}, I1{}, I7{});
     return hipGetLastError();
 }
@@ -340,9 +342,19 @@ bool stream_takes(const Launch &L, int maxM)
     const bool plain = L.fmt_a == Fmt::F16 && (L.epi == Epi::F16 || L.epi == Epi::F32);
     // Below K = 1024 a plain fp16 product's chain is short, and k_small_f16 takes most such products.
     if (plain && L.K < 1024) return false;
-    // One chain a wave serves 32 rows too, until the columns give the tiles half the CUs (20 x 4096 x 4096
-    // 13.5 us, tiles 22.1; 32 rows 15.4 and 22.3; at 8192 columns 32 x 2048 14.1 and 13.5).
-    const int most = one_chain(L) && (long)L.nprob * L.N < 8192 ? 32 : 16;
+    // Plain fp16 over columns whose 64-wide blocks nearly fill the CUs twice: more than 8 rows (16 x 5120 x 28672
+    // 77.8 us, tiles 63.0; 12 x 2560 x 28672 38.6 and 33.7; 16 x 2560 x 24576 0.91 of the tiles' time), 8 of long
+    // rows (8 x 5120 x 28672 1.11 of it).
+    if (one_chain(L) && L.nprob == 1 && L.N > 24576 && L.N <= 32768 && L.K >= 2560 && maxM > (L.K >= 4608 ? 4 : 8)) return false;
+    // Rows of 8 KB (one column block a wave, launch_chain) over columns short of a round of tiles: 16 x 4096 x
+    // 14336 30.1 us, tiles 26.2; 12 rows 27.9 and 26.3.
+    if (one_chain(L) && L.nprob == 1 && L.K == 4096 && L.N > 12288 && L.N < 16384 && maxM > 8) return false;
+    // One chain a wave serves 32 rows too, up to a wave a CU (20 x 4096 x 4096 13.5 us, tiles 22.1; 32 rows
+    // 15.4 and 22.3). Past it 20 rows, and more of short rows, until the columns give the tiles half the CUs
+    // (20 rows 1.03 to 1.16 of the tiles' rate at 5120 to 7936 columns, 32 rows 1.02 to 1.16 up to K = 1536,
+    // 0.97 at 2048, 0.90 at 8704; K = 12288, 20 rows 0.95).
+    const long cols = (long)L.nprob * L.N;
+    const int most = !one_chain(L) || cols >= 8192 ? 16 : cols <= 4096 || L.K <= 1536 ? 32 : L.K <= 8704 ? 20 : 16;
     // int8 weights: the tiles' chain is the shorter one a byte, and they win where their 64-column blocks
     // fill the CUs or rows are many and long (16 x 8192 x 16384 28.7 us, tiles 24.0; 4 x 4096 x 16384 14.5 and
     // 13.3; 16 x 8192 x 8192 16.5 and 15.2; one and a half rounds of tiles 4 x 8192 x 24576 1.16 times as

@@ -307,6 +307,18 @@ static void routes()
     // attention's results over V: V is copied first where its rows are no multiple of a tile
     CHECK(fa(1, 100, 64, 8, 8) && !ran("k_pad_cols"));
     CHECK(rocket_flash_attn_fp16(fd, 1, 100, 64, 64, 8, 8, 0.1f, 0.f, h(X), h(W), h(Y), nullptr, h(Y)) == 0 && ran("k_pad_cols"));
+    // plain fp16 over many columns, and 17 to 32 rows over more than a wave a CU
+    CHECK(fp16(fd, 16, 5120, 28672) == 0 && ran("k_gemm"));
+    CHECK(fp16(fd, 12, 2560, 28672) == 0 && ran("k_gemm"));
+    CHECK(fp16(fd, 8, 2560, 28672) == 0 && ran("k_chain"));
+    CHECK(fp16(fd, 16, 2560, 24576) == 0 && ran("k_chain"));
+    CHECK(fp16(fd, 16, 4096, 14336) == 0 && ran("k_gemm"));
+    CHECK(fp16(fd, 16, 4096, 16384) == 0 && ran("k_chain"));
+    CHECK(fp16(fd, 32, 4096, 4096) == 0 && ran("k_chain"));
+    CHECK(fp16(fd, 32, 8704, 7808) == 0 && ran("k_gemm"));
+    CHECK(fp16(fd, 20, 8704, 7808) == 0 && ran("k_chain"));
+    CHECK(fp16(fd, 20, 12288, 5120) == 0 && ran("k_gemm"));
+    CHECK(fp16(fd, 32, 1536, 5120) == 0 && ran("k_chain"));
     // fp16, 17 to 32 rows of short K
     CHECK(fp16(fd, 32, 992, 32768) == 0 && ran("k_small_f16"));
     CHECK(fp16(fd, 32, 992, 65536) == 0 && ran("k_gemm"));
