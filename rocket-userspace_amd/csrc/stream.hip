@@ -358,12 +358,13 @@ bool stream_takes(const Launch &L, int maxM)
     // int8 weights: the tiles' chain is the shorter one a byte, and they win where their 64-column blocks
     // fill the CUs or rows are many and long (16 x 8192 x 16384 28.7 us, tiles 24.0; 4 x 4096 x 16384 14.5 and
     // 13.3; 16 x 8192 x 8192 16.5 and 15.2; one and a half rounds of tiles 4 x 8192 x 24576 1.16 times as
-    // long), and on short rows from 32768 columns (4 x 512 x 32768 7.0 and 6.1; 4 x 2048 1.13 times as long).
+    // long, a little more than that 12 x 4224 x 25536 25.4 and 21.5; 16 x 4224 x 9216 0.94 of the tiles' rate, 12 x
+    // 4224 x 40960 0.87), and on short rows from 32768 columns (4 x 512 x 32768 7.0 and 6.1; 4 x 2048 1.13 times as long).
     if (L.fmt_b == Fmt::I8 && L.fmt_a == Fmt::I8) {
         const int blocks = (L.N + 63) / 64, last = blocks % 256;
-        if (L.K > 2048 && blocks >= 192 && (last == 0 || last >= 192)) return false;
+        if (L.K > 2048 && blocks >= 192 && (last == 0 || last >= 192 || (blocks > 256 && last > 128))) return false;
         if (L.K >= 256 && L.K < 2048 && blocks > 384) return false;
-        if ((long)maxM * L.K > 100000 && L.N > 4096) return false;
+        if ((long)maxM * L.K > (L.N > 32768 ? 50000 : L.N > 8192 ? 65000 : 100000) && L.N > 4096) return false;
     }
     // one K range, results written once; operand rows are addressed with 32-bit byte offsets (64 rows',
     // the smallest tile's: longer rows are refused by the tiled kernels' own check)

@@ -319,6 +319,13 @@ static void routes()
     CHECK(fp16(fd, 20, 8704, 7808) == 0 && ran("k_chain"));
     CHECK(fp16(fd, 20, 12288, 5120) == 0 && ran("k_gemm"));
     CHECK(fp16(fd, 32, 1536, 5120) == 0 && ran("k_chain"));
+    // int8 to int32 over a little more than whole rounds of tiles, and of many long rows
+    CHECK(int8(12, 4224, 25536) && ran("k_gemm"));
+    CHECK(int8(4, 4224, 22528) && ran("k_stream"));
+    CHECK(int8(16, 4224, 9216) && ran("k_gemm"));
+    CHECK(int8(12, 4224, 9216) && ran("k_stream"));
+    CHECK(int8(12, 4224, 40960) && ran("k_gemm"));
+    CHECK(int8(4, 4224, 40960) && ran("k_stream"));
     // fp16, 17 to 32 rows of short K
     CHECK(fp16(fd, 32, 992, 32768) == 0 && ran("k_small_f16"));
     CHECK(fp16(fd, 32, 992, 65536) == 0 && ran("k_gemm"));
