@@ -10,7 +10,8 @@
 // every workgroup) as the first, one set of steps in flight while the other's MFMAs run. The
 // waves' sums meet in LDS once, at the end, added in wave order. fp32 operands are truncated or
 // split in registers, so no conversion pass runs first. The K slices depend on the formats and
-// K alone: a row's bits do not depend on N, on M up to 16, or on the launch's other problems. Plain
+// K alone: a row's bits do not depend on N, on M, or on the launch's other problems where this kernel
+// runs (stream_takes leaves some of many columns to the tiles). Plain
 // fp16 products, whose rows have the tiled kernels' bits, take k_chain instead: one wave, all of K.
 //
 // Measured (three sets of operands in turn; tiled kernels before, this kernel after):
@@ -305,10 +306,24 @@ template <Fmt FA, Fmt FB, int KS> hipError_t launch_ks(SArgs &a, const Launch &L
     a.per = (a.nsteps + KS - 1) / KS;
     // 32 columns a workgroup (the activations' fragments shared by two column blocks) from one and a half
     // of them a CU. K = 3840, N = 15360: int4 16 rows 12.2 -> 9.5 us, 4 rows 8.5 -> 8.0; bf16 65.7 ->
-    // 52.9 and 47.0 -> 43.7; tf32, whose splitting it does not share, 66.4 -> 65.6 and 47.5 -> 61.0. At
-    // N = 4096, half a workgroup a CU, it loses: int4 4.9 -> 5.7 and 3.9 -> 4.9, bf16 16.1 -> 22.5 and
-    // 13.0 -> 19.0. (N = 8192 and 12288 go either way, 0.86 to 1.25 times.)
-    const bool glu = L.epi == Epi::GLU, wide = !glu && a.N >= 12288;
+    // 52.9 and 47.0 -> 43.7. At N = 4096, half a workgroup a CU, it loses: int4 4.9 -> 5.7 and 3.9 -> 4.9,
+    // bf16 16.1 -> 22.5 and 13.0 -> 19.0. (N = 8192 and 12288 go either way, 0.86 to 1.25 times.) fp32
+    // rows are twice the bytes in flight a column: tf32, which splits each of them, keeps 16 from K = 1024
+    // (4 x 3840 x 15360 47.5, wide 61.0; 8 x 3840 x 32768 105, 123), with more than 8 rows from K = 2048;
+    // bf16 keeps 16 at N = 12288 from K > 1024, and where its rows are a power of two of 8 KB and more, of
+    // which 32 at a time meet in the same channels (8 x 2048 x 12288 1.18 of the tiles' rate, wide 0.84; 4
+    // x 4096 x 20480 1.45 and 1.13; 12 x 6144 x 16384 0.89 and 1.09); it takes 32 with more than 12 rows where 16
+    // columns a workgroup are more than one a CU and less than two (16 x 6400 x 5120 0.90 and 1.18; 16 x 8192 x
+    // 6144 0.93 and 1.16).
+    const bool glu = L.epi == Epi::GLU;
+    bool wide = !glu && a.N >= 12288;
+    if (FB == Fmt::F32BF16 || FB == Fmt::F32TF32) {
+        int maxM = 0;
+        for (int i = 0; i < L.nprob; i++) maxM = std::max(maxM, a.M[i]);
+        if (FB == Fmt::F32TF32) wide = wide && a.N > 12288 && (a.K < 1024 || (a.K < 2048 && maxM > 8));
+        else wide = (wide && (a.K <= 1024 || (a.N > 12288 && (a.K < 2048 || (a.K & (a.K - 1)) != 0 || maxM > 12)))) ||
+                    (a.N > 4096 && a.N <= 8192 && (KS == 16 ? maxM > 8 : maxM > 12 && a.K >= 4096));
+    }
     const dim3 grid((unsigned)((a.N + (wide ? 31 : 15)) / (wide ? 32 : 16)), (unsigned)L.nprob);
     *blocks = (uint64_t)grid.x * grid.y;
     if (glu) {
@@ -366,6 +381,20 @@ bool stream_takes(const Launch &L, int maxM)
         if (L.K >= 256 && L.K < 2048 && blocks > 384) return false;
         if ((long)maxM * L.K > (L.N > 32768 ? 50000 : L.N > 8192 ? 65000 : 100000) && L.N > 4096) return false;
     }
+    // fp32 operands over many columns: the tiles on converted rows, whose 64-column blocks nearly fill the
+    // CUs there. bf16, 16 rows: from K = 2048 (16 x 3840 x 12288 49.9 us, tiles 46.9; 16 x 2048 x 14336 30.0 and
+    // 25.6; 16 x 3456 x 9216 38.0 and 34.2), but for K around 3072 (16 x 3072 x 20480 0.90 of the tiles' time); 12 rows at K = 2048; K = 8192 (8 x
+    // 8192 x 14336 114 and 104). tf32: at 32768 columns (16 x 3840 x 32768 129 and 97; 4 rows 94 and 96).
+    if (L.fmt_b == Fmt::F32BF16 && L.nprob == 1 && L.N > 8192 && L.N <= 28672 && L.K >= 1024) {
+        if (L.N > 24576) {
+            if (maxM > 8) return false;
+        } else if (L.K >= 2048) {
+            if (maxM > 12 && !(L.K >= 2560 && L.K < 3584 && L.N > 12288)) return false;
+            if (maxM > 8 && L.K < 2560 && L.N > 12288 && L.N <= 16384) return false;
+        }
+        if (L.K >= 8192 && L.N > 12288) return false;
+    }
+    if (L.fmt_b == Fmt::F32TF32 && L.nprob == 1 && L.N > 28672 && L.K >= 1024 && maxM > 4) return false;
     // one K range, results written once; operand rows are addressed with 32-bit byte offsets (64 rows',
     // the smallest tile's: longer rows are refused by the tiled kernels' own check)
     return maxM <= most && L.epi != Epi::GW && L.fmt_a != Fmt::I16 && !L.accum && L.kbeg == 0 && L.kend == L.K &&

@@ -326,6 +326,22 @@ static void routes()
     CHECK(int8(12, 4224, 9216) && ran("k_stream"));
     CHECK(int8(12, 4224, 40960) && ran("k_gemm"));
     CHECK(int8(4, 4224, 40960) && ran("k_stream"));
+    // fp32 operands, few rows over many columns
+    CHECK(bf16(fd, 16, 3840, 12288) == 0 && ran("k_gemm"));
+    CHECK(bf16(fd, 12, 3840, 12288) == 0 && ran("k_stream"));
+    CHECK(bf16(fd, 16, 3456, 9216) == 0 && ran("k_gemm"));
+    CHECK(bf16(fd, 16, 3072, 20480) == 0 && ran("k_stream"));
+    CHECK(bf16(fd, 12, 2048, 14336) == 0 && ran("k_gemm"));
+    CHECK(bf16(fd, 8, 8192, 14336) == 0 && ran("k_gemm"));
+    CHECK(tf32(16, 3840, 32768) && ran("k_gemm"));
+    CHECK(tf32(4, 3840, 32768) && ran("k_stream"));
+    // and their rows, converted ahead where tiles without K slices read them
+    CHECK(tf32(20, 3840, 14336) && ran("k_cvt"));
+    CHECK(tf32(100, 3840, 10240) && ran("k_cvt"));
+    CHECK(tf32(20, 1536, 7168) && ran("k_cvt"));
+    CHECK(tf32(1040, 256, 7792) && ran("k_cvt"));
+    CHECK(bf16(fd, 20, 3072, 10240) == 0 && ran("k_cvt"));
+    CHECK(bf16(fd, 20, 512, 32768) == 0 && ran("k_cvt"));
     // fp16, 17 to 32 rows of short K
     CHECK(fp16(fd, 32, 992, 32768) == 0 && ran("k_small_f16"));
     CHECK(fp16(fd, 32, 992, 65536) == 0 && ran("k_gemm"));
