@@ -37,8 +37,8 @@ int rocket_quantize_rows_int8_fp16(int fd, int M, int K, const _Float16 *A, int8
  * scales — the same bits as rocket_quantize_rows_int8 followed by
  * rocket_matmul_int{8,4}_prepacked_gw_rowscale, in one call (the int8 codes never leave the GPU).
  * Two launches; one, whose product quantises the rows itself, for few rows of moderate K (up to 16
- * rows and about 61440 elements in all, fewer where a workgroup has fewer waves or its LDS does not
- * hold them, and results not stored over the rows). This holds for every entry below that quantises.
+ * rows and 61440 elements in all, fewer where a workgroup has fewer waves or its LDS does not hold
+ * them, where that is expected to take less time, and results not stored over the rows). This holds for every entry below that quantises.
  * Same checks and return codes as the *_rowscale entry each mirrors. */
 int rocket_matmul_int8_prepacked_gw_f32in(rocket_i8_ctx *ctx, int M, int K, int N, const float *A,
                                           const float *b_scale, float *Cf, rocket_i8_weights *w);

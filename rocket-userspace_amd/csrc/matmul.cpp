@@ -191,7 +191,7 @@ int run(int fd, const Req &r)
     for (int p0 = 0; fuse && p0 < r.nprob; p0 += kMaxProblems) {
         Launch Lq;
         Lq.fmt_a = r.fa; Lq.fmt_b = fb_dev; Lq.epi = r.epi; Lq.N = r.N; Lq.K = Lq.kend = r.K;
-        Lq.group = r.group; Lq.kt = gw_period(r.group); Lq.rowscale = 1; Lq.qa = r.quant_a;
+        Lq.group = r.group; Lq.kt = gw_period(r.group); Lq.rowscale = 1; Lq.qa = r.quant_a; Lq.act = r.act;
         Lq.nprob = std::min(kMaxProblems, r.nprob - p0);
         int rows = 0;
         for (int q = 0; q < Lq.nprob; q++) rows += Lq.prob[q].M = r.M[p0 + q];

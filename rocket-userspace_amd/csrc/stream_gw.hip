@@ -418,26 +418,33 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
         g.split = g.lds <= lds && a.tiles <= 256 * (int)(lds / g.lds);
     }
     if (!g.split) {
-        // A wave a tile, W waves a workgroup that share the codes in LDS: the W whose busiest CU has
-        // the fewest tiles, a batch of workgroups that LDS does not hold beside the others counting
-        // as two (16 rows, 3840 x 15360: 11.9 us with four waves, 22.1 with two, which leave one
-        // workgroup a CU; the MoE's 1408 gate and up tiles: 29.1 with two, 35.1 with four).
+        // A wave a tile, W waves a workgroup that share the codes in LDS: the W of the least time, in
+        // half microseconds. A batch of workgroups that LDS holds together takes 20 and one for each of
+        // the busiest CU's waves (16 rows, 3840 x 15360: 11.9 us with four waves, 22.1 with two, which leave
+        // one workgroup a CU; 1408 gate and up tiles of 8 rows, K = 2048: 13.5 with two, 15.2 with eight, in
+        // one batch, 20.1 with four and 21.3 with one, in two; 1248 of 16, K = 1632: 11.8 with eight, 18.0 to
+        // 20.4 in two batches). Rows quantised here take e elements a thread in each batch, and more where
+        // they are formed from gate and up, of which 64 stay in registers (1344 tiles, 16 rows of 896: 22.4
+        // us with two waves, 12.9 with four, 10.8 with eight, 12.5 quantised ahead).
         a.depth = 3;
-        int best = 0, waves = 0, rounds = 0;   // of the best: waves a CU, batches of workgroups
+        int best = 0, ahead = 0, waves = 0, rounds = 0;   // of the best: waves a CU, batches of workgroups
         for (int w = 8; w >= 1; w /= 2) {
             const size_t b = shared + w * (tab + a.depth * slot);
             if (b > lds) continue;
             const int wgs = g.np * ((a.nbn + w - 1) / w), each = (wgs + 255) / 256, fit = (int)(lds / b);
-            const int cost = w * each + 2 * ((each + fit - 1) / fit);
+            const int batches = (each + fit - 1) / fit, e = L.K * (maxM <= 4 ? 4 : maxM <= 8 ? 8 : 16) / (64 * w);
+            const int plain = w * each + 20 * batches;
+            const int cost = plain + (!L.qa ? 0 : L.act ? batches * (e / 7 + (e > 64 ? 12 : 0)) : batches * e / 20);
+            if (!ahead || plain + 8 < ahead) ahead = plain + 8;
             if (!best || cost < best) {
                 best = cost;
                 g.w = w;
                 g.lds = b;
                 waves = w * fit;
-                rounds = (each + fit - 1) / fit;
+                rounds = batches;
             }
         }
-        if (!best) return false;
+        if (!best || (L.qa && ahead <= best)) return false;   // (a pass ahead takes 4 us)
         // Long rows leave LDS for one or two waves a CU, and several batches of those take longer than
         // the tiles: int4, from more batches than waves (16 x 8192 x 16384, groups of 128, one wave, four
         // batches: 90.6 us, tiles 44.2; 16 x 8192 x 12288, groups of 256, two and two: 38.1 and 33.4; 16 x

@@ -342,6 +342,28 @@ static void routes()
     CHECK(tf32(1040, 256, 7792) && ran("k_cvt"));
     CHECK(bf16(fd, 20, 3072, 10240) == 0 && ran("k_cvt"));
     CHECK(bf16(fd, 20, 512, 32768) == 0 && ran("k_cvt"));
+    // few-row group-wise launches of many tiles: as many waves a workgroup as make one batch of them, and
+    // rows quantised there only where that takes less than a pass ahead
+    auto moe = [&](int np, int M, int K, int N, int g, int qa) {
+        rk::Launch L;
+        L.fmt_a = L.fmt_b = rk::Fmt::I8; L.epi = rk::Epi::GW; L.N = N; L.K = L.kend = K;
+        L.group = L.kt = g; L.rowscale = 1; L.qa = qa; L.act = qa ? rk::kActSilu : 0;
+        L.nprob = np;
+        for (int i = 0; i < np; i++) L.prob[i] = rk::Problem{M, A, B, Y + 4096L * 4096 * i, X, W, nullptr};
+        for (int i = 0; qa && i < np; i++) L.prob[i].A2 = A;
+        uint64_t blocks = 0;
+        if (qa && !rk::gemm_quantises(L)) return uint64_t{0};
+        CHECK(rk::gemm_launch(L, &blocks) == hipSuccess);
+        fake::st().launches.clear();
+        return blocks;
+    };
+    CHECK(moe(16, 16, 1632, 1248, 32, 0) == 16 * 10);
+    CHECK(moe(16, 12, 3328, 1280, 128, 0) == 16 * 10);
+    CHECK(moe(16, 8, 2048, 1408, 32, 0) == 16 * 44);
+    CHECK(moe(8, 16, 896, 2688, 128, 2) == 8 * 21);
+    CHECK(moe(8, 12, 576, 2176, 32, 2) == 8 * 17);
+    CHECK(moe(8, 8, 1408, 2048, 32, 2) == 8 * 32);
+    CHECK(moe(8, 16, 1856, 3872, 32, 2) == 0);
     // fp16, 17 to 32 rows of short K
     CHECK(fp16(fd, 32, 992, 32768) == 0 && ran("k_small_f16"));
     CHECK(fp16(fd, 32, 992, 65536) == 0 && ran("k_gemm"));
