@@ -135,11 +135,12 @@ int f32_prepass(const Req &r)
     // 1024 x 8192 25.1 with it, 27.7 without; 2044 x 128 x 8192 35.7 and 42.2; 20 x 2048 x 16384 39.1 and
     // 48.3; 64 x 2048 x 8192 22 and 21.2; bf16, whose conversion in the loads is cheaper, 512 x 512 x
     // 16384 24.8 and 27.7; 64 x 4096 x 8192 35.0 and 45.5; 256 x 512 x 8192 13 and 12. tf32: where the
-    // tiles nearly fill the CUs no K slices shorten their chain, and the conversion is in it: 20 x 3840 x 14336
-    // 67.4 and 85.8, 100 x 3840 x 10240 71.2 and 87.2; in slices 20 x 3840 x 12288 0.94 of the time without;
-    // short rows of many: 1040 x 256 x 7792 36.5 and 42.3, 512 x 384 x 6144 0.94 of its rate without. bf16 at few rows: 20 x 3072 x 10240 31.0 and 36.6, 20 x 3840 x
-    // 20480 76.6 and 84.4, 100 x 1536 x 20480 32.1 and 39.2, 20 x 512 x 32768 21.6 and 23.6, 20 x 1024 x 24576
-    // 1.02 of the time without)
+    // tiles nearly fill the CUs no K slices shorten their chain, and the conversion is in it (20 x 3840 x
+    // 14336 67.4 us with it, 85.8 without, 100 x 3840 x 10240 71.2 and 87.2; in slices 20 x 3840 x 12288 is 1.06
+    // times as long with it); likewise where they are more than the CUs (1040 x 256 x 7792 36.5 and 42.3, 944 x
+    // 128 x 5312 19.8 and 21.9; 512 x 128 x 7792, in one round, 1.04 times as long with it). bf16, few
+    // rows: 20 x 3072 x 10240 31.0 and 36.6, 20 x 3840 x 20480 76.6 and 84.4, 100 x 1536 x 20480 32.1 and 39.2, 20 x
+    // 512 x 32768 21.6 and 23.6; 20 x 1024 x 24576 1.01 times as long with it)
     const long mk = (long)maxM * r.K, N = r.N, K = r.K;
     bool pays = N >= 384 && mk >= 400000;
     Launch L;   // the product on unconverted rows
@@ -147,7 +148,8 @@ int f32_prepass(const Req &r)
     L.nprob = 1;
     L.prob[0].M = maxM;
     if (r.fa == Fmt::F32TF32)
-        pays = pays || (N >= 4096 && ((K >= 64 && maxM > 1024) || (maxM >= 128 && mk * N >= 1000000000L))) || (K >= 256 && N > 16384) ||
+        pays = pays || (K >= 64 && (long)((maxM + 127) / 128) * ((N + 127) / 128) > 256) ||
+               (N >= 4096 && maxM >= 128 && mk * N >= 900000000L) || (K >= 256 && N > 16384) ||
                (N >= 6144 && K >= 512 && maxM > 128) ||
                (((N >= 8192 && K >= 512) || (N >= 3072 && K >= 1024)) && gemm_ws_bytes(L) == 0);
     else

@@ -340,6 +340,8 @@ static void routes()
     CHECK(tf32(100, 3840, 10240) && ran("k_cvt"));
     CHECK(tf32(20, 1536, 7168) && ran("k_cvt"));
     CHECK(tf32(1040, 256, 7792) && ran("k_cvt"));
+    CHECK(tf32(944, 128, 5312) && ran("k_cvt"));
+    CHECK(tf32(512, 128, 7792) && !ran("k_cvt"));
     CHECK(bf16(fd, 20, 3072, 10240) == 0 && ran("k_cvt"));
     CHECK(bf16(fd, 20, 512, 32768) == 0 && ran("k_cvt"));
     // few-row group-wise launches of many tiles: as many waves a workgroup as make one batch of them, and
