@@ -326,6 +326,10 @@ static void routes()
     CHECK(int8(12, 4224, 9216) && ran("k_stream"));
     CHECK(int8(12, 4224, 40960) && ran("k_gemm"));
     CHECK(int8(4, 4224, 40960) && ran("k_stream"));
+    // bf16 products that K slices of large tiles do not shorten
+    CHECK(bf16(fd, 652, 3328, 1728) == 0 && !ran("k_sum_slices"));
+    CHECK(bf16(fd, 320, 3776, 3536) == 0 && !ran("k_sum_slices"));
+    CHECK(bf16(fd, 384, 9408, 2048) == 0 && ran("k_sum_slices"));
     // fp32 operands, few rows over many columns
     CHECK(bf16(fd, 16, 3840, 12288) == 0 && ran("k_gemm"));
     CHECK(bf16(fd, 12, 3840, 12288) == 0 && ran("k_stream"));
