@@ -6,8 +6,9 @@
 // its 4 waves takes chunks of 32 keys and loads their K rows and V^T columns straight into
 // registers as MFMA fragments, 32 KB of them in flight a wave at head size 256, next chunk's K
 // while this chunk's scores and outputs are formed. All of a KV head's query rows share one
-// read of its keys. V^T rows of any length are read in place (an unaligned row costs nothing
-// here): no padded copy.
+// read of its keys. V^T rows of any length are read in place: no padded copy. (Rows at
+// 4-byte addresses cost nothing here; an odd number of keys, rows at 2-byte ones, up to twice the time of a
+// chunk.)
 //
 // Scores are transposed, S^T = K Q^T (v_mfma_f32_16x16x32_f16, K the first operand): lane l
 // holds query l % 16. The 16 rows of K block b are keys 8 (i / 4) + 4 b + i % 4, so that lane
@@ -60,26 +61,19 @@ struct RowArgs {
 };
 
 // Halves key .. key + 8 of a row of n (n >= 8), zeros past the row: the last eight are loaded
-// and shifted where the row ends inside.
+// and shifted where the row ends inside. No branch: one around each of a chunk's loads made them wait
+// for each other (1 x 255 keys in one workgroup a head, heads of 256: 20.8 -> 18.8 us).
 __device__ __forceinline__ i32x4 row8(const _Float16 *row, int key, int n)
 {
-    const int past = key + 8 - n;   // halves past the row's end
-    if (past >= 8) return i32x4{0, 0, 0, 0};
-    i32x4 v = reinterpret_cast<const Halves8 *>(row + (past > 0 ? n - 8 : key))->v;
-    if (past > 0) {
-        unsigned long lo = (unsigned)v[0] | ((unsigned long)(unsigned)v[1] << 32);
-        unsigned long hi = (unsigned)v[2] | ((unsigned long)(unsigned)v[3] << 32);
-        const int s = 16 * past;
-        if (s >= 64) {
-            lo = hi >> (s - 64);
-            hi = 0;
-        } else {
-            lo = (lo >> s) | (hi << (64 - s));
-            hi >>= s;
-        }
-        v = i32x4{(int)(unsigned)lo, (int)(lo >> 32), (int)(unsigned)hi, (int)(hi >> 32)};
-    }
-    return v;
+    const i32x4 v = reinterpret_cast<const Halves8 *>(row + min(key, n - 8))->v;
+    const int past = max(key + 8 - n, 0), s = 16 * (past & 3);   // halves past the row's end
+    unsigned long lo = (unsigned)v[0] | ((unsigned long)(unsigned)v[1] << 32);
+    unsigned long hi = (unsigned)v[2] | ((unsigned long)(unsigned)v[3] << 32);
+    lo = past >= 8 ? 0 : (past >= 4 ? hi : lo);
+    hi = past >= 4 ? 0 : hi;
+    lo = (lo >> s) | ((hi << 1) << (63 - s));
+    hi >>= s;
+    return i32x4{(int)(unsigned)lo, (int)(lo >> 32), (int)(unsigned)hi, (int)(hi >> 32)};
 }
 
 // Merges the splits, one (head, token) row a workgroup: out = sum_s w_s On_s / sum_s w_s with
@@ -314,11 +308,15 @@ template <int D> hipError_t launch_rows(const RowArgs &a, int kv_heads, hipStrea
 // Workgroups a KV head: one chunk a wave while the workgroups stay near three a CU; one workgroup for
 // short caches, where the merge's launch costs more than the waves' further chunks (one token, 32 heads
 // of 64, 192 keys 4.3 us, split 7.0; 512 keys 6.4 and 7.1; heads of 128, 320 keys 7.5 and 8.3, 384 keys
-// 8.1 and 8.3; heads of 256, 256 keys 10.2 and 10.5, 320 keys 12.2 and 10.5).
+// 8.1 and 8.3; heads of 256, 256 keys 10.2 and 10.5, 320 keys 12.2 and 10.5); fewer chunks with an odd
+// number of keys, whose loads take longer (heads of 64, 319 keys 7.7 and 8.1, 383 keys 8.7 and 8.3; heads of
+// 128, 255 keys 10.6 and 10.4, 319 keys 12.6 and 10.2; heads of 256, 159 keys 9.8 and 10.6, 191 keys 15.0
+// and 12.8, 255 keys 18.8 and 14.6).
 void split_of(const FaLaunch &L, int *nsplit, int *cps)
 {
     const int kvh = L.n_head / L.gqa, chunks = (L.n_kv + kChunk - 1) / kChunk;
-    const int d = std::max(L.dk, L.dv), whole = d <= 64 ? 16 : d <= 128 ? 10 : 8;
+    const int d = std::max(L.dk, L.dv), odd = L.n_kv & 1;
+    const int whole = d <= 64 ? (odd ? 10 : 16) : d <= 128 ? (odd ? 8 : 10) : odd ? 5 : 8;
     const int n = chunks <= whole ? 1 : std::min({(chunks + kWaves - 1) / kWaves, std::max(1, 768 / kvh), 64});
     *cps = (chunks + n - 1) / n;
     *nsplit = (chunks + *cps - 1) / *cps;

@@ -293,6 +293,11 @@ static void routes()
     CHECK(fa(1, 192, 128, 8, 8) && fake::st().launches.size() == 1 && ran("k_fa_rows"));
     CHECK(fa(1, 512, 64, 8, 8) && fake::st().launches.size() == 1 && ran("k_fa_rows"));
     CHECK(fa(1, 512, 128, 8, 8) && fake::st().launches.size() == 2 && ran("k_fa_rows"));
+    CHECK(fa(1, 256, 256, 8, 8) && fake::st().launches.size() == 1 && ran("k_fa_rows"));
+    CHECK(fa(1, 255, 256, 8, 8) && fake::st().launches.size() == 2 && ran("k_fa_rows"));
+    CHECK(fa(1, 159, 256, 8, 8) && fake::st().launches.size() == 1 && ran("k_fa_rows"));
+    CHECK(fa(1, 319, 128, 8, 8) && fake::st().launches.size() == 2 && ran("k_fa_rows"));
+    CHECK(fa(1, 511, 64, 8, 8) && fake::st().launches.size() == 2 && ran("k_fa_rows"));
     CHECK(fa(1, 8192, 256, 32, 32) && ran("k_flash_attn"));
     CHECK(fa(1, 8191, 256, 32, 32) && ran("k_fa_rows"));
     CHECK(fa(1, 8192, 256, 64, 32) && ran("k_fa_rows"));
