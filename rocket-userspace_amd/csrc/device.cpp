@@ -224,12 +224,14 @@ void Call::want(const void *p, size_t bytes)
     if (!direct_(p)) need_ += round_(bytes);
 }
 
-bool Call::capturing_()
+bool stream_capturing(hipStream_t s)
 {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(h_->stream, &cap) != hipSuccess) (void)hipGetLastError();
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
     return cap != hipStreamCaptureStatusNone;
 }
+
+bool Call::capturing_() { return stream_capturing(h_->stream); }
 
 size_t Call::want_optional(size_t bytes, bool worth)
 {

@@ -54,6 +54,9 @@ bool is_device_ptr(const void *p, int device);
 // Stages one call's operands. in()/out() return the device address the kernel uses:
 // the caller's own pointer when it is 16-byte-aligned device memory, otherwise a slice
 // of the handle's arena (inputs copied in, results copied back by finish()).
+// Whether the stream is being captured into a graph.
+bool stream_capturing(hipStream_t s);
+
 class Call {
 public:
     Call(Handle *h, const char *who) : h_(h), who_(who) {}

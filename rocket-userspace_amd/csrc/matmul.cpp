@@ -174,8 +174,15 @@ int run(int fd, const Req &r)
     const bool gw = (r.epi == Epi::GW);
     // B as it arrives from the caller: int8 per value when we pack it ourselves
     const size_t brow_in = r.pack_b_int4 ? (size_t)r.K : fmt_row_bytes(r.fb, r.K);
-    const int prepass = f32_prepass(r);
+    int prepass = f32_prepass(r);
     const Fmt cvt = r.fa == Fmt::F32TF32 ? Fmt::BF16X2 : Fmt::BF16;
+    // (a capture cannot grow the arena for converted rows: the product converts them as it loads them, the
+    // same bits, unless its results lie over them)
+    if (prepass == 2) {
+        size_t rows = 0;
+        for (int p = 0; p < r.nprob; p++) rows += ((size_t)std::max(r.M[p], 0) * fmt_row_bytes(cvt, r.K) + 255) & ~(size_t)255;
+        if (rows > L.h->arena_cap && stream_capturing(L.h->stream) && !results_overlap_rows(r, (size_t)r.K * 4, 4)) prepass = 0;
+    }
     const Fmt fa_dev = prepass ? cvt : r.fa;
     const Fmt fb_dev = r.pack_b_int4 ? Fmt::I4P : (prepass == 1 ? cvt : r.fb);
 

@@ -119,6 +119,21 @@ static void small_calls_hold_no_scratch()
     rocket_close(fd);
 }
 
+// fp32 rows that are converted ahead are converted in the product where a captured call has no arena for them.
+static void rows_converted_without_an_arena()
+{
+    const int fd = open_async();
+    auto tf32 = [&] { return rocket_matmul_tf32(fd, 20, 3840, 14336, X, W, Y); };
+    auto bf = [&] { return bf16(fd, 16, 3840, 12288); };
+    CHECK(captured(tf32).size() == 1);
+    CHECK(captured(bf).size() == 1);
+    CHECK(captured([&] { return bf16(fd, 20, 3072, 10240); }).size() == 1);
+    fake::st().launches.clear();
+    CHECK(tf32() == 0 && fake::count("k_cvt") == 1);
+    CHECK(captured(tf32).size() == 2);
+    rocket_close(fd);
+}
+
 // A block's second product runs without its K slices where the arena holds the hidden rows alone.
 static void blocks_on_a_small_arena()
 {
@@ -427,6 +442,7 @@ int main()
 {
     arena_kept_for_graphs();
     small_calls_hold_no_scratch();
+    rows_converted_without_an_arena();
     blocks_on_a_small_arena();
     short_of_memory();
     dumps_run_the_same_kernel();
