@@ -67,6 +67,7 @@ struct Launch {
     int act = 0;              // GLU / ACT, or qa with A2: kActSilu or kActGelu
     int qa = 0;               // GW, rowscale: A holds fp32 (1) or fp16 (2) rows, quantised per row in the kernel
                               // (quant_rows' formula; only where gemm_quantises says so)
+    int qa_must = 0;          // with qa: also where quantising them ahead is expected to take less time
     int free_sums = 0;        // plain fp16: 1, K may be summed in any slices (a block's own product); 0, the slices
                               // depend on the tiles' plan for M > 128 alone, so that a row's bits do not depend
                               // on the launch's other problems, nor, up to 128 rows, on M

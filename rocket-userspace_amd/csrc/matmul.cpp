@@ -196,11 +196,16 @@ int run(int fd, const Req &r)
     const size_t a_row_in = qa_bytes ? qa_bytes * r.K : fmt_row_bytes(r.fa, r.K);
 
     // few rows: the product quantises them itself (every launch of the call, or none)
+    // (where that is the shorter way, or a capture cannot grow the arena for the codes)
+    size_t codes = 0;
+    for (int p = 0; p < r.nprob; p++) codes += (size_t)std::max(r.M[p], 0) * (r.K + sizeof(float));
+    const int must = qa_bytes && codes > L.h->arena_cap && stream_capturing(L.h->stream);
     bool fuse = qa_bytes != 0;
     for (int p0 = 0; fuse && p0 < r.nprob; p0 += kMaxProblems) {
         Launch Lq;
         Lq.fmt_a = r.fa; Lq.fmt_b = fb_dev; Lq.epi = r.epi; Lq.N = r.N; Lq.K = Lq.kend = r.K;
         Lq.group = r.group; Lq.kt = gw_period(r.group); Lq.rowscale = 1; Lq.qa = r.quant_a; Lq.act = r.act;
+        Lq.qa_must = must;
         Lq.nprob = std::min(kMaxProblems, r.nprob - p0);
         int rows = 0;
         for (int q = 0; q < Lq.nprob; q++) rows += Lq.prob[q].M = r.M[p0 + q];
@@ -293,6 +298,7 @@ int run(int fd, const Req &r)
         Lc.rowscale = r.rowscale;
         Lc.f16out = r.f16out ? 1 : 0;
         Lc.qa = fuse ? r.quant_a : 0;
+        Lc.qa_must = must;
         Lc.act = fuse ? r.act : 0;
         Lc.kt = gw ? gw_period(r.group) : 0;
         Lc.ws = wsp;

@@ -430,7 +430,7 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
         int best = 0, ahead = 0, waves = 0, rounds = 0;   // of the best: waves a CU, batches of workgroups
         for (int w = 8; w >= 1; w /= 2) {
             const size_t b = shared + w * (tab + a.depth * slot);
-            if (b > lds) continue;
+            if (b > lds || (L.qa_must && (long)maxM * L.K > 120L * w * 64)) continue;
             const int wgs = g.np * ((a.nbn + w - 1) / w), each = (wgs + 255) / 256, fit = (int)(lds / b);
             const int batches = (each + fit - 1) / fit, e = L.K * (maxM <= 4 ? 4 : maxM <= 8 ? 8 : 16) / (64 * w);
             const int plain = w * each + 20 * batches;
@@ -444,7 +444,7 @@ bool plan_gw(const Launch &L, int maxM, GPlan &g, GArgs &a)
                 rounds = batches;
             }
         }
-        if (!best || (L.qa && ahead <= best)) return false;   // (a pass ahead takes 4 us)
+        if (!best || (L.qa && !L.qa_must && ahead <= best)) return false;   // (a pass ahead takes 4 us)
         // Long rows leave LDS for one or two waves a CU, and several batches of those take longer than
         // the tiles: int4, from more batches than waves (16 x 8192 x 16384, groups of 128, one wave, four
         // batches: 90.6 us, tiles 44.2; 16 x 8192 x 12288, groups of 256, two and two: 38.1 and 33.4; 16 x

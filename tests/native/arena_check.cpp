@@ -134,6 +134,37 @@ static void rows_converted_without_an_arena()
     rocket_close(fd);
 }
 
+// Rows that are quantised ahead are quantised in the product where a captured call has no arena for the codes.
+static void rows_quantised_without_an_arena()
+{
+    const int fd = open_async();
+    const std::vector<int> M(8, 12);
+    const std::vector<const void *> A(8, X), A2(8, X + 500000), B(8, W);
+    const std::vector<const float *> S(8, W + 10000000);
+    std::vector<void *> C;
+    for (int i = 0; i < 8; i++) C.push_back(Y + 100000 * i);
+    rk::Req r;
+    r.epi = rk::Epi::GW;
+    r.K = 1344;
+    r.N = 2560;
+    r.nprob = 8;
+    r.M = M.data();
+    r.A = A.data();
+    r.A2 = A2.data();
+    r.B = B.data();
+    r.C = C.data();
+    r.b_scale = S.data();
+    r.group = 32;
+    r.rowscale = true;
+    r.quant_a = 1;
+    r.act = rk::kActSilu;
+    for (int n = 1024; n <= 6144; n += 512) {   // (fused by the estimate, or not)
+        r.N = n;
+        CHECK(captured([&] { return rk::run(fd, r); }).size() == 1);
+    }
+    rocket_close(fd);
+}
+
 // A block's second product runs without its K slices where the arena holds the hidden rows alone.
 static void blocks_on_a_small_arena()
 {
@@ -443,6 +474,7 @@ int main()
     arena_kept_for_graphs();
     small_calls_hold_no_scratch();
     rows_converted_without_an_arena();
+    rows_quantised_without_an_arena();
     blocks_on_a_small_arena();
     short_of_memory();
     dumps_run_the_same_kernel();
